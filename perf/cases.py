@@ -336,8 +336,10 @@ def _dipole_octant(ext, cell, accuracy=6):
     d = [torch.clamp(a - 1, min=0) * c for a, c in zip(g, cell)]
     dist = torch.sqrt(d[0] ** 2 + d[1] ** 2 + d[2] ** 2).reshape(-1)
     dist[dist == 0] = min(cell)
-    size = dist / accuracy
-    num = torch.stack([(torch.clamp(c / size, min=1.0) + 0.5).to(torch.int64) for c in cell])
+    # divisions by tensors: by a number they are products with its inverse, and the point counts jump where the
+    # quotient is a half
+    size = dist / torch.full_like(dist, accuracy)
+    num = torch.stack([(torch.clamp(torch.full_like(size, c) / size, min=1.0) + 0.5).to(torch.int64) for c in cell])
     R = [a.reshape(-1) * c for a, c in zip(g, cell)]
     key = (num[0] * 4096 + num[1]) * 4096 + num[2]
     out = torch.zeros(6, dist.numel(), device=dev, dtype=f8)

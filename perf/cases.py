@@ -7,6 +7,7 @@ that is resident on the GPU, as a simulation script has it:
             the table's <m>; returns m and <m>
     field   Sim.update of H_eff or of the torque at a new m; returns the field
     batch   Batch.steps(count) of uneven films; returns every m
+    plan    construction of a demag plan and its first field
     kernels one field evaluation and RK stage composed from the drop-in
             kernels, as an engine on the C entry points composes it
     train   one training step of the learned demag correction; returns the
@@ -47,11 +48,10 @@ def listed():
     return [
         # the standard-problem film: the smallest grid people run, bound by launches and latency
         _case(name="film_128x32x1_rk12", nx=128, ny=32, cell=3.90625, bext=0.01, count=20),
-        # a film on round decimal sizes (500 nm x 125 nm): lengths with factors of 5
-        _case(name="film_500x125x1_rk12", nx=500, ny=125, cell=1.0, cellz=3.0, bext=0.02, count=10),
-        # a slab on decimal sizes under a spin-polarised current
-        _case(name="slab_100x100x10_zhangli_rk12", nx=100, ny=100, nz=10, cell=2.5, cellz=2.5, zl=True,
-              alpha=0.1, count=10),
+        # a film on round decimal sizes (500 nm x 125 nm) under a spin-polarised current: lengths with factors of 5
+        _case(name="film_500x125x1_zhangli_rk12", nx=500, ny=125, cell=1.0, cellz=3.0, zl=True, count=10),
+        # what every script waits for first: the demag kernel of its grid, up to the first field
+        _case(name="plan_200x200x5_first_field", kind="plan", nx=200, ny=200, nz=5),
         # ragged, periodic along x, patterned (geometry mask and exchange map): the torque for a relaxation check
         _case(name="ragged_96x70x11_torque", kind="field", nx=96, ny=70, nz=11, pbc_x=1, disk=True, aex_map=True,
               quantity="torque"),
@@ -88,7 +88,7 @@ def _smooth(rng, lo, hi, even=False):
 
 
 def draw(rng):
-    kind = rng.choices(("steps", "field", "kernels", "batch", "train"), (45, 30, 10, 10, 5))[0]
+    kind = rng.choices(("steps", "field", "plan", "kernels", "batch", "train"), (42, 28, 8, 9, 8, 5))[0]
     c = _case(kind=kind, cell=rng.choice((1.0, 2.0, 2.5, 4.0, 5.0)), cellz=rng.choice((2.0, 3.0, 4.0)),
               msat=round(rng.uniform(6e5, 1.2e6)), alpha=round(rng.uniform(0.01, 0.2), 4))
     if kind == "batch":
@@ -97,7 +97,7 @@ def draw(rng):
     if kind == "train":
         c.update(nx=16 * rng.randint(4, 16), ny=16 * rng.randint(4, 16), nz=rng.randint(1, 5), cell=4.0)
         return c
-    most = 1 << 23 if kind == "field" else 1 << 22
+    most = {"field": 1 << 23, "plan": 200000}.get(kind, 1 << 22)
     while True:
         nx, ny = _smooth(rng, 16, 1024, even=True), _smooth(rng, 16, 1024, even=True)
         nz = 1 if rng.random() < 0.35 else _smooth(rng, 2, 64)
@@ -107,6 +107,8 @@ def draw(rng):
              disk=rng.random() < 0.3, zl=rng.random() < 0.3)
     if rng.random() < 0.25:
         c[rng.choice(("pbc_x", "pbc_y"))] = 1
+    if kind == "plan":
+        c.update(cell=4.0, cellz=rng.choice((3.0, 4.0)), ku=0.0, bext=0.0, disk=False, zl=False, pbc_x=0, pbc_y=0)
     if kind == "field":
         c.update(quantity=rng.choice(("H_eff", "H_eff", "torque")), aex_map=rng.random() < 0.2)
     if kind == "steps":
@@ -232,6 +234,9 @@ def prepare(case, seed):
     if case["kind"] == "batch":
         sims = [_sim(c, c["seed"]) for c in _films(case, seed)]
         return {"case": case, "sims": sims, "batch": mmx.Batch(sims)}
+    if case["kind"] == "plan":
+        m = _texture(_n(case), seed)
+        return {"case": case, "m": m, "b": torch.zeros_like(m)}
     if case["kind"] == "kernels":
         n = _n(case)
         z = lambda: torch.zeros((3,) + n, device="cuda")  # noqa: E731
@@ -264,6 +269,11 @@ def run(state):
     if kind == "field":
         state["sim"].update(case["quantity"])
         return {case["quantity"]: state["out"]}
+    if kind == "plan":
+        plan = mmx.DemagPlan(_n(case), _cell(case), _pbc(case))
+        plan.update_b(state["b"].data_ptr(), state["m"].data_ptr(), case["msat"], None,
+                      torch.cuda.current_stream().cuda_stream)
+        return {"B": state["b"]}
     if kind == "batch":
         state["batch"].steps(case["count"])
         return {"m": [_view(s, "m") for s in state["sims"]]}
@@ -318,6 +328,8 @@ def work(case):
         return {"bytes": b * case["count"], "flops": f * 2 * case["count"]}
     if kind == "field":
         return {"bytes": b + (4.0 * cells if case["disk"] else 0) + (4.0 * cells if case["aex_map"] else 0), "flops": f}
+    if kind == "plan":      # per displacement and source axis: 4 points' pairs of poles at least, in 64 bits
+        return {"bytes": b, "flops": f + 3 * 4 * 50.0 * 8 * cells}
     if kind == "kernels":   # m and the mask in; H_eff, torque and the predictor out
         return {"bytes": b + 28.0 * cells, "flops": f + 120.0 * cells}
     pixels = case["nx"] * case["ny"]    # forward, backward-data and weight gradients of four 3x3 layers
@@ -530,8 +542,10 @@ def exact(case, seed):
             out.append(e.m)
         return {"m": out}
     e = _Exact(case, seed)
-    if kind == "kernels":   # m as it is given, not normalised first
+    if kind in ("plan", "kernels"):     # m as it is given, not normalised first
         e.m = _texture(e.n, seed).double() * (1.0 if e.mask is None else e.mask)
+    if kind == "plan":
+        return {"B": MU0 * e.demag(e.m)}
     if kind == "steps":
         for _ in range(case["count"]):
             e.step()

@@ -7,6 +7,7 @@
 // The kernel is then transformed with an FP64 FFT (the reference uses a float32
 // cuFFT here, maxwell_convolution.go:386-396), the real part of the octant
 // kz <= p0/2, ky <= p1/2, kx <= p2/2 is kept and scaled by 1/(p0 p1 p2).
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <vector>
@@ -25,7 +26,7 @@ struct ArneArgs {
     int x1, x2, y1, y2, z1, z2;
     double L;
     double accuracy;
-    int s;
+    int reach[3];   // displacements within it are in arne_near's table
 };
 
 __device__ inline double delta_cells(int d)
@@ -45,87 +46,206 @@ __device__ inline int first_image(int w, int p, int lo)
     return x;
 }
 
-// B (FP64) at displacement (x, y, z) of a unit s-dipole: the surface-charge /
-// volume integration of kernel_magnetostatic.go:94-165, same operations in the
-// same order.
-__device__ inline void arne_point(const ArneArgs &a, int x, int y, int z, double Bf[3])
-{
-    const int X = 0, Y = 1, Z = 2;
-    const double *cell = a.cell;
-    const int s = a.s;
-    const int u = s, v = (s + 1) % 3, w = (s + 2) % 3;
-    double R[3], R2[3], pole[3];
-    R[X] = (double)x * cell[X];
-    R[Y] = (double)y * cell[Y];
-    R[Z] = (double)z * cell[Z];
+// The quadrature of one displacement of a unit S-dipole: the point counts,
+// first point and spacing per axis, and the charge of one point
+// (kernel_magnetostatic.go:94-146).  The source axis is a template argument so
+// that every index is a constant (registers, not scratch).
+template <int S> struct ArneQuad {
+    static constexpr int U = S, V = (S + 1) % 3, W = (S + 2) % 3;
+    int nv, nw, n[3];
+    double v0, dv, w0, dw;   // face points: v0 + i dv, w0 + j dw
+    double r0[3], dr[3];     // destination points: r0 + dr k
+    double charge, pu1, pu2;
+};
 
-    const double dx = delta_cells(x) * cell[X];
-    const double dy = delta_cells(y) * cell[Y];
-    const double dz = delta_cells(z) * cell[Z];
+template <int S>
+__device__ inline ArneQuad<S> arne_quad(const ArneArgs &a, int x, int y, int z)
+{
+    using Q = ArneQuad<S>;
+    const double *cell = a.cell;
+    Q q;
+    const double R[3] = {(double)x * cell[0], (double)y * cell[1], (double)z * cell[2]};
+    const double dx = delta_cells(x) * cell[0];
+    const double dy = delta_cells(y) * cell[1];
+    const double dz = delta_cells(z) * cell[2];
     double d = sqrt(dx * dx + dy * dy + dz * dz);
     if (d == 0) d = a.L;
     const double maxSize = d / a.accuracy;
-    int nv = (int)(fmax(cell[v] / maxSize, 1.) + 0.5);
-    int nw = (int)(fmax(cell[w] / maxSize, 1.) + 0.5);
-    const int nx_ = (int)(fmax(cell[X] / maxSize, 1.) + 0.5);
-    const int ny_ = (int)(fmax(cell[Y] / maxSize, 1.) + 0.5);
-    const int nz_ = (int)(fmax(cell[Z] / maxSize, 1.) + 0.5);
-    nv *= 2;
-    nw *= 2;
-    const double scale = 1 / (double)(nv * nw * nx_ * ny_ * nz_);
-    const double surface = cell[v] * cell[w];
-    const double charge = surface * scale;
-    const double pu1 = cell[u] / 2.;
-    const double pu2 = -pu1;
+#pragma unroll
+    for (int c = 0; c < 3; c++) q.n[c] = (int)(fmax(cell[c] / maxSize, 1.) + 0.5);
+    q.nv = 2 * q.n[Q::V];
+    q.nw = 2 * q.n[Q::W];
+    const double scale = 1 / (double)(q.nv * q.nw * q.n[0] * q.n[1] * q.n[2]);
+    const double surface = cell[Q::V] * cell[Q::W];
+    q.charge = surface * scale;
+    q.pu1 = cell[Q::U] / 2.;
+    q.pu2 = -q.pu1;
+    q.v0 = -(cell[Q::V] / 2.) + cell[Q::V] / (double)(2 * q.nv);
+    q.dv = cell[Q::V] / (double)q.nv;
+    q.w0 = -(cell[Q::W] / 2.) + cell[Q::W] / (double)(2 * q.nw);
+    q.dw = cell[Q::W] / (double)q.nw;
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+        q.r0[c] = R[c] - cell[c] / 2. + cell[c] / (double)(2 * q.n[c]);
+        q.dr[c] = cell[c] / (double)q.n[c];
+    }
+    return q;
+}
 
+// Field of the two charged face points (i, j) at the point (k0, k1, k2) of the
+// destination cell: the term that kernel_magnetostatic.go:128-165 adds to B,
+// same operations in the same order.
+template <int S>
+__device__ inline void arne_term(const ArneQuad<S> &q, int i, int j, int k0, int k1, int k2,
+                                 double t[3])
+{
+    using Q = ArneQuad<S>;
+    double R2[3], pole[3], b[3];
+    pole[Q::V] = q.v0 + (double)i * q.dv;
+    pole[Q::W] = q.w0 + (double)j * q.dw;
+    const double rc[3] = {q.r0[0] + q.dr[0] * (double)k0, q.r0[1] + q.dr[1] * (double)k1,
+                          q.r0[2] + q.dr[2] * (double)k2};
+    pole[Q::U] = q.pu1;
+#pragma unroll
+    for (int c = 0; c < 3; c++) R2[c] = rc[c] - pole[c];
+    double r = sqrt(R2[0] * R2[0] + R2[1] * R2[1] + R2[2] * R2[2]);
+    double qr = q.charge / (4. * kPi * r * r * r);
+#pragma unroll
+    for (int c = 0; c < 3; c++) b[c] = R2[c] * qr;
+    pole[Q::U] = q.pu2;
+    R2[Q::U] = rc[Q::U] - pole[Q::U];
+    r = sqrt(R2[0] * R2[0] + R2[1] * R2[1] + R2[2] * R2[2]);
+    qr = -q.charge / (4. * kPi * r * r * r);
+#pragma unroll
+    for (int c = 0; c < 3; c++) t[c] = b[c] + R2[c] * qr;
+}
+
+// B (FP64) at displacement (x, y, z) of a unit S-dipole: the surface-charge /
+// volume integration of kernel_magnetostatic.go:94-165, its terms added in the
+// reference's loop order.
+template <int S>
+__device__ inline void arne_point(const ArneArgs &a, int x, int y, int z, double Bf[3])
+{
+    const ArneQuad<S> q = arne_quad<S>(a, x, y, z);
     Bf[0] = Bf[1] = Bf[2] = 0.0;
-    for (int i = 0; i < nv; i++) {
-        const double pv = -(cell[v] / 2.) + cell[v] / (double)(2 * nv) + (double)i * (cell[v] / (double)nv);
-        pole[v] = pv;
-        for (int j = 0; j < nw; j++) {
-            const double pw = -(cell[w] / 2.) + cell[w] / (double)(2 * nw) + (double)j * (cell[w] / (double)nw);
-            pole[w] = pw;
-            for (int al = 0; al < nx_; al++) {
-                const double rx = R[X] - cell[X] / 2. + cell[X] / (double)(2 * nx_) + (cell[X] / (double)nx_) * (double)al;
-                for (int be = 0; be < ny_; be++) {
-                    const double ry = R[Y] - cell[Y] / 2. + cell[Y] / (double)(2 * ny_) + (cell[Y] / (double)ny_) * (double)be;
-                    for (int ga = 0; ga < nz_; ga++) {
-                        const double rz = R[Z] - cell[Z] / 2. + cell[Z] / (double)(2 * nz_) + (cell[Z] / (double)nz_) * (double)ga;
-                        pole[u] = pu1;
-                        R2[X] = rx - pole[X];
-                        R2[Y] = ry - pole[Y];
-                        R2[Z] = rz - pole[Z];
-                        double r = sqrt(R2[X] * R2[X] + R2[Y] * R2[Y] + R2[Z] * R2[Z]);
-                        double qr = charge / (4. * kPi * r * r * r);
-                        const double bx = R2[X] * qr;
-                        const double by = R2[Y] * qr;
-                        const double bz = R2[Z] * qr;
-                        pole[u] = pu2;
-                        R2[X] = rx - pole[X];
-                        R2[Y] = ry - pole[Y];
-                        R2[Z] = rz - pole[Z];
-                        r = sqrt(R2[X] * R2[X] + R2[Y] * R2[Y] + R2[Z] * R2[Z]);
-                        qr = -charge / (4. * kPi * r * r * r);
-                        Bf[X] += (bx + R2[X] * qr);
-                        Bf[Y] += (by + R2[Y] * qr);
-                        Bf[Z] += (bz + R2[Z] * qr);
+    for (int i = 0; i < q.nv; i++)
+        for (int j = 0; j < q.nw; j++)
+            for (int al = 0; al < q.n[0]; al++)
+                for (int be = 0; be < q.n[1]; be++)
+                    for (int ga = 0; ga < q.n[2]; ga++) {
+                        double t[3];
+                        arne_term<S>(q, i, j, al, be, ga, t);
+                        for (int c = 0; c < 3; c++) Bf[c] += t[c];
                     }
+}
+
+// The displacements |x_a| <= reach[a], whose quadratures have more than the
+// four points of the far field (up to (2 accuracy)^2 accuracy^3 and more where
+// the cells are not cubes), are integrated beforehand, one workgroup each:
+// wave 0 adds the terms one after another in the loop order of arne_point (so
+// the sum has the same bits) while the other eight waves work out the next 512.
+// A single thread's serial chain of square roots and divisions took 15 ms per
+// source axis for cubic cells (31104 points per displacement at accuracy 6), 27
+// for 4x4x3 nm (98304) and 640 for 8x8x3 nm; here the chain is the additions,
+// 6 ns each: all three axes of 4x4x3 nm in 0.60 ms (1.39 ms when the adding
+// wave waited for the LDS at every second term).
+constexpr int kNearWaves = 8;
+constexpr int kNearChunk = 64 * kNearWaves;
+
+template <int S>
+__device__ __forceinline__ void arne_near_one(const ArneArgs &a, float *__restrict__ tab,
+                                              double (&buf)[2][3][kNearChunk])
+{
+    const int e1 = 2 * a.reach[1] + 1, e2 = 2 * a.reach[2] + 1;
+    const int x = (int)blockIdx.x / (e1 * e2) - a.reach[0];
+    const int y = (int)blockIdx.x / e2 % e1 - a.reach[1];
+    const int z = (int)blockIdx.x % e2 - a.reach[2];
+    const ArneQuad<S> q = arne_quad<S>(a, x, y, z);
+    // the point's indices as digits (i, j, al, be, ga), advanced by one chunk
+    // at a time with carries (no division per point)
+    const int base[4] = {q.n[2], q.n[1], q.n[0], q.nw};
+    const long npts = (long)q.nv * q.nw * q.n[0] * q.n[1] * q.n[2];
+    const long nchunk = (npts + kNearChunk - 1) / kNearChunk;
+    const int lane = threadIdx.x;
+    int dig[5], step[5];
+    for (int part = 0; part < 2; part++) {
+        int r = part ? kNearChunk : lane - 64;
+        int *d = part ? step : dig;
+        for (int c = 0; c < 4; c++) {
+            d[c] = r % base[c];
+            r /= base[c];
+        }
+        d[4] = r;
+    }
+    double B = 0.0;
+    for (long k = 0; k <= nchunk; k++) {
+        if (lane >= 64 && k < nchunk) {
+            const int e = lane - 64;
+            if (k * kNearChunk + e < npts) {
+                double t[3];
+                arne_term<S>(q, dig[4], dig[3], dig[2], dig[1], dig[0], t);
+                for (int c = 0; c < 3; c++) buf[k & 1][c][e] = t[c];
+            }
+            int carry = 0;
+            for (int c = 0; c < 4; c++) {
+                dig[c] += step[c] + carry;
+                carry = dig[c] >= base[c] ? 1 : 0;
+                dig[c] -= carry ? base[c] : 0;
+            }
+            dig[4] += step[4] + carry;
+        }
+        if (lane < 3 && k > 0) {
+            const double *t = buf[(k - 1) & 1][lane];
+            const long left = npts - (k - 1) * kNearChunk;
+            if (left >= kNearChunk) {
+                // 16 terms ahead in registers: the additions wait for each
+                // other, not for the LDS
+                double now[16], next[16];
+#pragma unroll
+                for (int e = 0; e < 16; e++) now[e] = t[e];
+                for (int at = 16; at <= kNearChunk; at += 16) {
+                    const double *tn = t + (at < kNearChunk ? at : 0);
+#pragma unroll
+                    for (int e = 0; e < 16; e++) next[e] = tn[e];
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int e = 0; e < 16; e++) B += now[e];
+#pragma unroll
+                    for (int e = 0; e < 16; e++) now[e] = next[e];
                 }
+            } else {
+                for (int e = 0; e < (int)left; e++) B += t[e];
             }
         }
+        __syncthreads();
+    }
+    if (lane < 3) tab[3 * ((size_t)S * gridDim.x + blockIdx.x) + lane] = (float)B;
+}
+
+__global__ void __launch_bounds__(64 + kNearChunk) __attribute__((amdgpu_waves_per_eu(3, 3)))
+arne_near(ArneArgs a, float *__restrict__ tab)
+{
+    __shared__ double buf[2][3][kNearChunk];
+    switch (blockIdx.y) {
+    case 0: arne_near_one<0>(a, tab, buf); break;
+    case 1: arne_near_one<1>(a, tab, buf); break;
+    default: arne_near_one<2>(a, tab, buf); break;
     }
 }
 
-// One thread per padded-grid element (xw, yw, zw): the element is the float32
-// sum, starting from 0, of float32(B) over every displacement (x, y, z) in the
+// One thread per padded-grid element (xw, yw, zw) and source axis: the element
+// is the float32 sum, starting from 0, of float32(B) over every displacement (x, y, z) in the
 // loop ranges that wraps onto it, added in the reference's loop order (x, then
 // y, then z ascending; kernel_magnetostatic.go:91-101,168-172).  Without
 // periodic images an element has at most one displacement; with them the
 // element is the same float32 sum the reference forms, with no atomics, so the
 // kernel is deterministic and bit-identical to it.  Every element is written.
-__global__ void __launch_bounds__(kBlock) arne_kernel(ArneArgs a, float *__restrict__ K6)
+// Near displacements come from arne_near's table.
+__global__ void __launch_bounds__(kBlock) arne_kernel(ArneArgs a, const float *__restrict__ tab,
+                                                      float *__restrict__ K6)
 {
     const int X = 0, Y = 1, Z = 2;
+    const int s = blockIdx.y;
     const long P = (long)a.p[X] * a.p[Y] * a.p[Z];
     const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= P) return;
@@ -135,17 +255,49 @@ __global__ void __launch_bounds__(kBlock) arne_kernel(ArneArgs a, float *__restr
     const int xs = first_image(xw, a.p[X], a.x1);
     const int ys = first_image(yw, a.p[Y], a.y1);
     const int zs = first_image(zw, a.p[Z], a.z1);
+    const int *r = a.reach;
+    const int e0 = 2 * r[0] + 1, e1 = 2 * r[1] + 1, e2 = 2 * r[2] + 1;
     float acc[3] = {0.0f, 0.0f, 0.0f};
     for (int x = xs; x <= a.x2; x += a.p[X])
         for (int y = ys; y <= a.y2; y += a.p[Y])
             for (int z = zs; z <= a.z2; z += a.p[Z]) {
+                if (abs(x) <= r[0] && abs(y) <= r[1] && abs(z) <= r[2]) {
+                    const size_t d = ((size_t)(x + r[0]) * e1 + (y + r[1])) * e2 + (z + r[2]);
+                    const float *b = tab + 3 * ((size_t)s * e0 * e1 * e2 + d);
+                    for (int dd = 0; dd < 3; dd++) acc[dd] += b[dd];
+                    continue;
+                }
                 double Bf[3];
-                arne_point(a, x, y, z, Bf);
+                switch (s) {
+                case 0: arne_point<0>(a, x, y, z, Bf); break;
+                case 1: arne_point<1>(a, x, y, z, Bf); break;
+                default: arne_point<2>(a, x, y, z, Bf); break;
+                }
                 for (int dd = 0; dd < 3; dd++) acc[dd] += (float)Bf[dd];
             }
     for (int dd = 0; dd < 3; dd++) {
-        const int idx = kStoredIdx[a.s][dd];
+        const int idx = kStoredIdx[s][dd];
         if (idx >= 0) K6[idx * P + t] = acc[dd];
+    }
+}
+
+// Reach of the near table per axis: an axis is cut into more than one piece
+// while cell / (d / accuracy) >= 1.5 for the largest cell, d measured from
+// one cell on.  Limited to the grid's displacements, and to 2^20 of them in
+// all (an accuracy in the hundreds): the rest is integrated element by element.
+static void arne_reach(ArneArgs &a)
+{
+    const int most[3] = {a.x2 > -a.x1 ? a.x2 : -a.x1, a.y2 > -a.y1 ? a.y2 : -a.y1,
+                         a.z2 > -a.z1 ? a.z2 : -a.z1};
+    const double far = a.accuracy * fmax(a.cell[0], fmax(a.cell[1], a.cell[2])) / 1.5;
+    for (double d = far;; d *= 0.8) {
+        double count = 1.0;
+        for (int c = 0; c < 3; c++) {
+            const double cells = floor(d / a.cell[c]) + 1.0;
+            a.reach[c] = cells < (double)most[c] ? (int)cells : most[c];
+            count *= 2.0 * a.reach[c] + 1.0;
+        }
+        if (count <= (double)(1 << 20)) return;
     }
 }
 
@@ -266,7 +418,7 @@ __global__ void __launch_bounds__(kBlock) newell_octant(NewellArgs a, double *__
 // odd in both of their axes.  Optionally also the float32 copy (real_f32).
 __global__ void __launch_bounds__(kBlock) newell_expand(const double *__restrict__ oct, int e0, int e1,
                                                         int e2, int p0, int p1, int p2, int c,
-                                                        double2 *__restrict__ full,
+                                                        double *__restrict__ real,
                                                         float *__restrict__ real_f32)
 {
     const long P = (long)p0 * p1 * p2;
@@ -290,7 +442,7 @@ __global__ void __launch_bounds__(kBlock) newell_expand(const double *__restrict
                 if (disp[bx] < 0) v = -v;
             }
         }
-        full[t] = double2{v, 0.0};
+        real[t] = v;
         if (real_f32) real_f32[t] = (float)v;
     }
 }
@@ -334,37 +486,85 @@ static void newell_rule5(double t[5], double w[5])
 }
 
 // max |x| of a float array into *dst (bits of a non-negative float)
+// (component blockIdx.y of n floats)
 __global__ void __launch_bounds__(kBlock) maxabs_kernel(const float *__restrict__ a, long n,
                                                         unsigned int *dst)
 {
+    a += blockIdx.y * n;
+    dst += blockIdx.y;
     float m = 0.0f;
     for (long t = (long)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += (long)gridDim.x * blockDim.x)
         m = fmaxf(m, fabsf(a[t]));
     block_max_to(m, dst);
 }
 
-__global__ void __launch_bounds__(kBlock) real_to_complex_f64(const float *__restrict__ a, long n,
-                                                              double2 *__restrict__ z)
-{
-    for (long t = (long)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += (long)gridDim.x * blockDim.x)
-        z[t] = double2{(double)a[t], 0.0};
-}
+// FP64 transform of the kernel, one component at a time.  The spectrum of a
+// real kernel is kept as its half kx <= p2/2 (rows of h2 points), and the octant
+// needs only ky <= p1/2 of the y transform's output, so the passes run over
+// all rows along x, over kx < h2 along y and over ky < nky, kx < h2 along z.  A
+// workgroup takes W neighbouring lines (consecutive in memory for y and z,
+// 16 W bytes of each row); with one line per workgroup and every line of the
+// full complex grid these passes took 3.0 ms at 200x200x5, here 0.41 ms.
 
-// In-place FP64 FFT of every line along one axis; the element t of a line is
-// at base + t*inner.  One line per workgroup (one-time use, not hot).
-__global__ void __launch_bounds__(kBlock) axis_fft_f64(double2 *__restrict__ data, long inner,
-                                                       LineFFT<double> f)
+// x: row r of the real input (float32 kernel, or FP64 for Newell's) -> h2 points
+template <typename T>
+__global__ void __launch_bounds__(kBlock) x_fft_f64(const T *__restrict__ a, long nrows, int W, int h2,
+                                                    double2 *__restrict__ out, LineFFT<double> f)
 {
     extern __shared__ double2 smd[];
-    const int L = f.L;
-    double2 *A = smd, *B = smd + L;
-    const long line = blockIdx.x;
-    const long outer = line / inner, in = line - outer * inner;
-    double2 *base = data + outer * inner * L + in;
-    for (int t = threadIdx.x; t < L; t += blockDim.x) A[t] = base[(long)t * inner];
+    const int L = f.L, ls = L + 1;
+    double2 *A = smd, *B = smd + W * ls;
+    const long row0 = (long)blockIdx.x * W;
+    for (int t = threadIdx.x; t < W * L; t += blockDim.x) {
+        const int r = t / L, k = t - r * L;
+        A[r * ls + k] = double2{row0 + r < nrows ? (double)a[row0 * L + t] : 0.0, 0.0};
+    }
     __syncthreads();
-    const double2 *R = lds_fft<double, -1>(A, B, 1, L, 1, f);
-    for (int t = threadIdx.x; t < L; t += blockDim.x) base[(long)t * inner] = R[t];
+    const double2 *R = lds_fft<double, -1>(A, B, W, ls, 1, f);
+    for (int t = threadIdx.x; t < W * h2; t += blockDim.x) {
+        const int r = t / h2, k = t - r * h2;
+        if (row0 + r < nrows) out[row0 * h2 + t] = R[r * ls + k];
+    }
+}
+
+// y or z, in place: line (o, q), o = blockIdx.y < outer planes, q < nline, has
+// its element t at o * L * inner + t * inner + q
+__global__ void __launch_bounds__(kBlock) axis_fft_f64(double2 *__restrict__ data, long inner,
+                                                       long nline, int W, LineFFT<double> f)
+{
+    extern __shared__ double2 smd[];
+    const int L = f.L, ls = L + 1;
+    double2 *A = smd, *B = smd + W * ls;
+    const long q0 = (long)blockIdx.x * W;
+    double2 *base = data + (long)blockIdx.y * L * inner + q0;
+    for (int e = threadIdx.x; e < W * L; e += blockDim.x) {
+        const int t = e / W, w = e - t * W;
+        A[w * ls + t] = q0 + w < nline ? base[t * inner + w] : double2{0.0, 0.0};
+    }
+    __syncthreads();
+    const double2 *R = lds_fft<double, -1>(A, B, W, ls, 1, f);
+    for (int e = threadIdx.x; e < W * L; e += blockDim.x) {
+        const int t = e / W, w = e - t * W;
+        if (q0 + w < nline) base[t * inner + w] = R[w * ls + t];
+    }
+}
+
+// lines per workgroup: two buffers of W lines within 48 KB, at most 8 (128-byte
+// pieces of a row); one line of up to 4096 points takes 131 KB
+static int fft_f64_lines(int L)
+{
+    int w = 8;
+    while (w > 1 && 2ull * w * (L + 1) * sizeof(double2) > 48 * 1024) w /= 2;
+    return w;
+}
+
+static size_t fft_f64_lds(int L) { return 2ull * fft_f64_lines(L) * (L + 1) * sizeof(double2); }
+
+template <typename K> static void allow_lds_f64(K kernel, size_t bytes)
+{
+    if (bytes > 65536)
+        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
 }
 
 __global__ void __launch_bounds__(kBlock) zero_strided(float *__restrict__ out, long n)
@@ -374,8 +574,8 @@ __global__ void __launch_bounds__(kBlock) zero_strided(float *__restrict__ out, 
 }
 
 // Octant extraction with the 1/Np scale; realness statistics over it.
-__global__ void __launch_bounds__(kBlock) extract_octant(const double2 *__restrict__ full, int p0,
-                                                         int p1, int p2, int ko0, int ko1,
+__global__ void __launch_bounds__(kBlock) extract_octant(const double2 *__restrict__ full,
+                                                         int p1, int ko0, int ko1,
                                                          int h2, double inv,
                                                          float *__restrict__ out,
                                                          unsigned int *maxbad,
@@ -387,7 +587,7 @@ __global__ void __launch_bounds__(kBlock) extract_octant(const double2 *__restri
         const int kx = (int)(t % h2);
         const int ky = (int)((t / h2) % ko1);
         const int kz = (int)(t / ((long)h2 * ko1));
-        const double2 v = full[((long)kz * p1 + ky) * p2 + kx];
+        const double2 v = full[((long)kz * p1 + ky) * h2 + kx];
         out[6 * t] = (float)(v.x * inv); // component slot of `out` set by the caller
         bad = fmaxf(bad, (float)fabs(v.y));
         good = fmaxf(good, (float)fabs(v.x));
@@ -402,8 +602,8 @@ __global__ void __launch_bounds__(kBlock) extract_octant(const double2 *__restri
 // 0, YZ and XY in axis 1).  For a kernel given by the caller this maximum
 // deviation of the full FP64 spectrum from that rule is checked.
 __global__ void __launch_bounds__(kBlock) octant_mirror_dev(const double2 *__restrict__ full,
-                                                            int p0, int p1, int p2, int h2,
-                                                            int odd0, int odd1,
+                                                            int p0, int p1, int h2, int odd0,
+                                                            int odd1,
                                                             unsigned int *maxdev)
 {
     const long n = (long)p0 * p1 * h2;
@@ -416,8 +616,8 @@ __global__ void __launch_bounds__(kBlock) octant_mirror_dev(const double2 *__res
         if (!mz && !my) continue;
         const int kzp = mz ? p0 - kz : kz, kyp = my ? p1 - ky : ky;
         const double sign = ((mz && odd0) ? -1.0 : 1.0) * ((my && odd1) ? -1.0 : 1.0);
-        const double a = full[((long)kz * p1 + ky) * p2 + kx].x;
-        const double b = full[((long)kzp * p1 + kyp) * p2 + kx].x;
+        const double a = full[((long)kz * p1 + ky) * h2 + kx].x;
+        const double b = full[((long)kzp * p1 + kyp) * h2 + kx].x;
         dev = fmaxf(dev, (float)fabs(a - sign * b));
     }
     block_max_to(dev, maxdev);
@@ -514,8 +714,10 @@ int build_demag_kernel(DemagPlanImpl *P, bool keep_real)
                 "the Newell kernel supports non-periodic grids only");
 
     float *K6 = nullptr;     // Arne: float32 real-space kernel (6 x Pn); Newell: kept copy
+    float *tab = nullptr;    // Arne: near-field table
     double *oct = nullptr;   // Newell: FP64 octant table (6 per displacement)
-    double2 *full = nullptr;
+    double *real64 = nullptr; // Newell: one component of the padded real-space kernel
+    double2 *full = nullptr; // one component's half spectrum (p0 x p1 x h2)
     unsigned int *stats = nullptr;
     void *twd = nullptr;
     int rc = MMX_OK;
@@ -529,11 +731,13 @@ int build_demag_kernel(DemagPlanImpl *P, bool keep_real)
     hipError_t err = hipSuccess;
     if (!newell || keep_real) err = hipMalloc(&K6, sizeof(float) * 6 * Pn);
     if (err == hipSuccess && newell) err = hipMalloc(&oct, sizeof(double) * 6 * ne);
-    if (err == hipSuccess) err = hipMalloc(&full, sizeof(double2) * Pn);
+    if (err == hipSuccess && newell) err = hipMalloc(&real64, sizeof(double) * Pn);
+    if (err == hipSuccess) err = hipMalloc(&full, sizeof(double2) * (size_t)p[0] * p[1] * g.h2);
     if (err == hipSuccess) err = hipMalloc(&stats, sizeof(unsigned int) * 16);
     if (err != hipSuccess) {
         (void)hipFree(K6);
         (void)hipFree(oct);
+        (void)hipFree(real64);
         (void)hipFree(full);
         (void)hipFree(stats);
         set_error("kernel build: cannot allocate the FP64 work arrays (%ld points)", Pn);
@@ -565,8 +769,7 @@ int build_demag_kernel(DemagPlanImpl *P, bool keep_real)
                               hipMemcpyHostToDevice) != hipSuccess) { fail(MMX_ERR_HIP); break; }
             }
             if (rc) break;
-            for (int c = 0; c < 6; c++)
-                maxabs_kernel<<<dim3(gb), dim3(kBlock)>>>(K6 + c * Pn, Pn, stats + c);
+            maxabs_kernel<<<dim3(gb, 6), dim3(kBlock)>>>(K6, Pn, stats);
             if (hipGetLastError() != hipSuccess) { set_error("maxabs launch failed"); fail(MMX_ERR_HIP); break; }
         } else {
             // ranges of Kernel_Arne (kernel_magnetostatic.go:50-65)
@@ -587,20 +790,23 @@ int build_demag_kernel(DemagPlanImpl *P, bool keep_real)
             if (P->cell[2] < L) L = P->cell[2];
             a.L = L;
             a.accuracy = (double)P->accuracy;
-            for (int s = 0; s < 3; s++) {
-                a.s = s;
-                arne_kernel<<<dim3(div_up(Pn, kBlock)), dim3(kBlock)>>>(a, K6);
-                if (hipGetLastError() != hipSuccess) { set_error("arne_kernel launch failed"); fail(MMX_ERR_HIP); break; }
+            arne_reach(a);
+            const int near = (2 * a.reach[0] + 1) * (2 * a.reach[1] + 1) * (2 * a.reach[2] + 1);
+            if (hipMalloc(&tab, sizeof(float) * 9 * (size_t)near) != hipSuccess) {
+                set_error("kernel build: cannot allocate the near-field table (%d displacements)", near);
+                fail(MMX_ERR_NOMEM);
+                break;
             }
-            if (rc) break;
+            arne_near<<<dim3(near, 3), dim3(64 + kNearChunk)>>>(a, tab);
+            arne_kernel<<<dim3(div_up(Pn, kBlock), 3), dim3(kBlock)>>>(a, tab, K6);
+            if (hipGetLastError() != hipSuccess) { set_error("arne_kernel launch failed"); fail(MMX_ERR_HIP); break; }
             if (P->dex) {
                 dex_combine<<<dim3(4096), dim3(kBlock)>>>(K6, Pn, P->dex_ms, P->dex_cex,
                                                           exch6_points(p, P->cell));
                 if (hipGetLastError() != hipSuccess) { set_error("dex_combine launch failed"); fail(MMX_ERR_HIP); break; }
             }
             // IsZero test per component (maxwell_convolution.go:412-418)
-            for (int c = 0; c < 6; c++)
-                maxabs_kernel<<<dim3(gb), dim3(kBlock)>>>(K6 + c * Pn, Pn, stats + c);
+            maxabs_kernel<<<dim3(gb, 6), dim3(kBlock)>>>(K6, Pn, stats);
             if (hipGetLastError() != hipSuccess) { set_error("maxabs launch failed"); fail(MMX_ERR_HIP); break; }
         }
         unsigned int hs[16];
@@ -627,12 +833,11 @@ int build_demag_kernel(DemagPlanImpl *P, bool keep_real)
             f[ax].tw = (const double2 *)twd + off[ax];
         }
         if (rc) break;
-        for (int ax = 0; ax < 3; ax++) {
-            const size_t b = 2 * sizeof(double2) * p[ax];
-            if (b > 65536)
-                (void)hipFuncSetAttribute(reinterpret_cast<const void *>(axis_fft_f64),
-                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)b);
-        }
+        allow_lds_f64(x_fft_f64<float>, fft_f64_lds(p[2]));
+        allow_lds_f64(x_fft_f64<double>, fft_f64_lds(p[2]));
+        allow_lds_f64(axis_fft_f64, std::max(fft_f64_lds(p[1]), fft_f64_lds(p[0])));
+        // the caller's kernel: every ky, for the symmetry check
+        const int nky = P->host_kernel ? p[1] : g.ko1;
 
         const long octant = (long)g.ko0 * g.ko1 * g.h2;
         const double inv = 1.0 / (double)Pn;
@@ -649,26 +854,29 @@ int build_demag_kernel(DemagPlanImpl *P, bool keep_real)
                 if (hipGetLastError() != hipSuccess) { set_error("kernel zero launch failed"); fail(MMX_ERR_HIP); break; }
                 continue;
             }
-            if (newell)
+            const long nrows = (long)p[0] * p[1];
+            const int wx = fft_f64_lines(p[2]), wy = fft_f64_lines(p[1]), wz = fft_f64_lines(p[0]);
+            if (newell) {
                 newell_expand<<<dim3(4096), dim3(kBlock)>>>(oct, e[0], e[1], e[2], p[0], p[1], p[2], c,
-                                                            full, K6 ? K6 + c * Pn : nullptr);
-            else
-                real_to_complex_f64<<<dim3(4096), dim3(kBlock)>>>(K6 + c * Pn, Pn, full);
-            long inner = 1;
-            for (int ax = 2; ax >= 0; ax--) {
-                if (p[ax] > 1) {
-                    const size_t b = 2 * sizeof(double2) * p[ax];
-                    axis_fft_f64<<<dim3((unsigned)(Pn / p[ax])), dim3(kBlock), b>>>(full, inner, f[ax]);
-                }
-                inner *= p[ax];
+                                                            real64, K6 ? K6 + c * Pn : nullptr);
+                x_fft_f64<double><<<dim3(div_up(nrows, wx)), dim3(kBlock), fft_f64_lds(p[2])>>>(
+                    real64, nrows, wx, g.h2, full, f[2]);
+            } else {
+                x_fft_f64<float><<<dim3(div_up(nrows, wx)), dim3(kBlock), fft_f64_lds(p[2])>>>(
+                    K6 + c * Pn, nrows, wx, g.h2, full, f[2]);
             }
-            extract_octant<<<dim3(1024), dim3(kBlock)>>>(full, p[0], p[1], p[2], g.ko0, g.ko1, g.h2,
-                                                         inv, dst, stats + 8, stats + 9);
+            axis_fft_f64<<<dim3(div_up(g.h2, wy), p[0]), dim3(kBlock), fft_f64_lds(p[1])>>>(
+                full, g.h2, g.h2, wy, f[1]);
+            if (p[0] > 1)
+                axis_fft_f64<<<dim3(div_up((long)nky * g.h2, wz), 1), dim3(kBlock), fft_f64_lds(p[0])>>>(
+                    full, (long)p[1] * g.h2, (long)nky * g.h2, wz, f[0]);
+            extract_octant<<<dim3(1024), dim3(kBlock)>>>(full, p[1], g.ko0, g.ko1, g.h2, inv, dst,
+                                                         stats + 8, stats + 9);
             if (P->host_kernel) {
                 // components XX,YY,ZZ,YZ,XZ,XY: odd in axis 0 for XZ, XY; in axis 1 for YZ, XY
                 const int odd0 = (c == 4 || c == 5), odd1 = (c == 3 || c == 5);
-                octant_mirror_dev<<<dim3(1024), dim3(kBlock)>>>(full, p[0], p[1], p[2], g.h2, odd0,
-                                                                odd1, stats + 10);
+                octant_mirror_dev<<<dim3(1024), dim3(kBlock)>>>(full, p[0], p[1], g.h2, odd0, odd1,
+                                                                stats + 10);
             }
             if (hipGetLastError() != hipSuccess) { set_error("kernel FFT launch failed"); fail(MMX_ERR_HIP); break; }
         }
@@ -701,7 +909,9 @@ int build_demag_kernel(DemagPlanImpl *P, bool keep_real)
         K6 = nullptr;
     }
     (void)hipFree(K6);
+    (void)hipFree(tab);
     (void)hipFree(oct);
+    (void)hipFree(real64);
     (void)hipFree(full);
     (void)hipFree(stats);
     (void)hipFree(twd);

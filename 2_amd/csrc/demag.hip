@@ -10,6 +10,11 @@
 //   XI  C2R along x, only k < n2 kept, fused with exchange, anisotropy,
 //       Zeeman, the LLG/Zhang-Li torque and the RK stage update.
 // For p0 == 1 (films) YF/Z/YI collapse into one kernel.
+// Each pass has three forms: register four-step kernels per length
+// (demag_fast.hip), composite-radix kernels for every other length whose prime
+// factors are at most 13 and for the x passes of small grids (comp_x.hip,
+// comp_y.hip, comp_z.hip), and the kernels of this file, one stage per prime
+// factor above 7, for the remaining lengths.
 // Replaces MaxwellPlan.update (maxwell_convolution.go:272-309): zeroing,
 // CopyPad3D, 3 cuFFT R2C, 9 cmadd passes, 3 cuFFT C2R and CopyUnPad3D.
 #include <atomic>
@@ -58,16 +63,6 @@ z_kernel(DemagGeom g, LineFFT<float> fz, int W, const float *__restrict__ K,
 {
     extern __shared__ float2 sm[];
     z_tile(g, fz, W, blockIdx.x * W, blockIdx.y, K, yb, sm);
-}
-
-// short z (z_small_applies): one thread per spectrum column
-__global__ void __launch_bounds__(kBlock)
-z_small_kernel(DemagGeom g, const float *__restrict__ K, float2 *__restrict__ yb)
-{
-    const long col = (long)blockIdx.x * kBlock + threadIdx.x;
-    if (col >= (long)g.p1 * g.h2) return;
-    const int ky = (int)(col / g.h2), kx = (int)(col - (long)ky * g.h2);
-    z_column_small_any(g, K, yb, ky, kx);
 }
 
 // ---------------------------------------------- film pass: y, multiply, y^-1
@@ -149,6 +144,11 @@ static int y_and_z_passes(DemagPlanImpl *P, hipStream_t st)
         mark(P, st, PASS_Y2D);
         return MMX_OK;
     }
+    if (g.p0 == 1 && comp_y2d_applies(P)) {
+        MMX_TRY(comp_y2d(P, st));
+        mark(P, st, PASS_Y2D);
+        return MMX_OK;
+    }
     if (g.p0 == 1) {
         const size_t b = lds_bytes_y(P, 3);
         allow_lds(y2d_kernel, b);
@@ -159,6 +159,9 @@ static int y_and_z_passes(DemagPlanImpl *P, hipStream_t st)
     }
     if (P->fast_y) {
         MMX_TRY(fast_yf(P, st));
+        mark(P, st, PASS_YF);
+    } else if (comp_y_applies(P)) {
+        MMX_TRY(comp_yf(P, st));
         mark(P, st, PASS_YF);
     } else {
         const size_t b = lds_bytes_y(P, 1);
@@ -171,10 +174,8 @@ static int y_and_z_passes(DemagPlanImpl *P, hipStream_t st)
     if (P->fast_z) {
         MMX_TRY(fast_z(P, st));
         mark(P, st, PASS_Z);
-    } else if (z_small_applies(g)) {
-        z_small_kernel<<<dim3((unsigned)div_up((long)g.p1 * g.h2, kBlock)), dim3(kBlock), 0, st>>>(
-            g, P->kern, P->ybuf);
-        MMX_CHECK_LAUNCH();
+    } else if (comp_z_applies(P)) {
+        MMX_TRY(comp_z(P, st));
         mark(P, st, PASS_Z);
     } else {
         const int ntx_z = div_up(g.h2, P->tiles.w_z);
@@ -187,6 +188,9 @@ static int y_and_z_passes(DemagPlanImpl *P, hipStream_t st)
     }
     if (P->fast_y) {
         MMX_TRY(fast_yi(P, st));
+        mark(P, st, PASS_YI);
+    } else if (comp_y_applies(P)) {
+        MMX_TRY(comp_yi(P, st));
         mark(P, st, PASS_YI);
     } else {
         const size_t b = lds_bytes_y(P, 1);
@@ -222,6 +226,8 @@ int demag_forward(DemagPlanImpl *P, const float *m, const float *msat_map, hipSt
     mark(P, st, PASS_START);
     if (fast_xf_used(P)) {
         MMX_TRY(fast_xf(P, 0, m, msat_map, nullptr, 0.0f, nullptr, nullptr, st));
+    } else if (comp_x_applies(P)) {
+        MMX_TRY(comp_xf(P, 0, m, msat_map, nullptr, 0.0f, nullptr, nullptr, st));
     } else {
         xf_kernel<0><<<dim3(nb), dim3(kBlock), b, st>>>(g, P->fx, P->tiles.rows_x, m, msat_map,
                                                          nullptr, 0.0f, nullptr, nullptr, P->xbuf,
@@ -244,6 +250,8 @@ int demag_forward_pred(DemagPlanImpl *P, const float *m0, const float *tau0, flo
     mark(P, st, PASS_START);
     if (fast_xf_used(P)) {
         MMX_TRY(fast_xf(P, 1, m0, norm_map, tau0, h, norm_map, mpred, st));
+    } else if (comp_x_applies(P)) {
+        MMX_TRY(comp_xf(P, 1, m0, norm_map, tau0, h, norm_map, mpred, st));
     } else {
         xf_kernel<1><<<dim3(nb), dim3(kBlock), b, st>>>(g, P->fx, P->tiles.rows_x, m0, norm_map,
                                                          tau0, h, norm_map, mpred, P->xbuf, nullptr,
@@ -264,6 +272,11 @@ int demag_inverse(DemagPlanImpl *P, int mode, const FieldParams &fp, const Epilo
     const int pass_xi = (g.p0 == 1) ? 2 : 4;
     if (P->fast_x && fast_x_blocks(g) >= fast_x_min_blocks()) {
         MMX_TRY(fast_xi(P, mode, fp, io, st));
+        mark(P, st, pass_xi);
+        return MMX_OK;
+    }
+    if (comp_x_applies(P)) {
+        MMX_TRY(comp_xi(P, mode, fp, io, st));
         mark(P, st, pass_xi);
         return MMX_OK;
     }

@@ -76,7 +76,9 @@ int fast_z(const DemagPlanImpl *P, hipStream_t st)
 // p1) of a grid with a single ky; the film's octant (ky, kx) then sits where
 // the z pass reads (kz, 0, kx), with the kz stride h2 (ko1 := 1); the
 // mirror of the transformed axis then negates YZ and XY (film_y), not XZ and
-// XY as along internal axis 0.
+// XY as along internal axis 0.  At length 2048 its two-column tiles of 192
+// threads take 88 us (1024x1024x1), the composite-radix pass, with 768 threads
+// and half the registers, 76: that length goes there.
 bool fast_y2d_as_z_applies(const DemagGeom &g)
 {
     DemagGeom f = g;
@@ -85,7 +87,7 @@ bool fast_y2d_as_z_applies(const DemagGeom &g)
     f.p1 = 1;
     f.ko0 = g.ko1;
     f.ko1 = 1;
-    return g.p0 == 1 && fast_length(g.p1) && fast_z_addressable(f);
+    return g.p0 == 1 && g.p1 <= 1024 && fast_length(g.p1) && fast_z_addressable(f);
 }
 
 int fast_y2d_as_z(const DemagPlanImpl *P, hipStream_t st)

@@ -17,6 +17,33 @@ struct DemagGeom {
     long nrows;        // n0 n1
 };
 
+// Quotients by a run-time divisor d < 2^16 of numbers below 2^16 (tasks and
+// elements of one workgroup): (x ceil(2^32 / d)) >> 32.
+struct FastDiv {
+    unsigned d = 1, mul = 0;
+    __host__ void set(int v)
+    {
+        d = (unsigned)v;
+        mul = v > 1 ? (unsigned)((0x100000000ull + (unsigned)v - 1) / (unsigned)v) : 0u;
+    }
+    __device__ __forceinline__ int quot(int x) const
+    {
+        return mul ? (int)__umulhi((unsigned)x, mul) : x;
+    }
+};
+
+// One length's composite-radix transform (comp_fft.hpp), L = R0 R1 (R2): radices
+// and the quotients its kernels need.
+struct CompFFT {
+    int L = 0, ns = 0;            // stages; 0: the length has no such plan
+    int R[3] = {1, 1, 1};
+    int Rl = 1, P = 1, Ml = 1;    // last radix, its odd pitch in the LDS, L / Rl
+    FastDiv byM[3];               // L / R[s]: tasks per line of stage s
+    FastDiv byL, byRl, byR0, byR1, byMl;
+    const float2 *tw = nullptr;   // L twiddles, forward sign
+    const float2 *rtw = nullptr;  // R2C split factors (x)
+};
+
 // What the last (C2R) pass does with the demag field of each cell.
 enum EpilogueMode : int {
     EPI_B = 0,      // out = demag_scale * conv (B in tesla, or H)
@@ -109,6 +136,8 @@ struct DemagPlanImpl {
     // demagexch kernel build: real-space kernel Ms K_d + dex_cex K_ex
     bool dex = false;
     double dex_ms = 0, dex_cex = 0;
+    // composite-radix transforms of the x half-length, y and z (ns = 0: none)
+    CompFFT cx, cy, cz;
 };
 
 // Pass names in launch order (3-D grids; films run xf, y2d, xi).
@@ -146,6 +175,31 @@ int fast_yi(const DemagPlanImpl *P, hipStream_t st);
 int fast_x_blocks(const DemagGeom &g);
 bool fast_y2d_as_z_applies(const DemagGeom &g);
 int fast_y2d_as_z(const DemagPlanImpl *P, hipStream_t st);
+// Radices of length L (comp_x.hip): two stages with radices up to top2 if
+// possible, else three with radices up to 32; the first radix is the largest.
+// ns = 0: L has a prime factor above 13, or no such split.
+CompFFT comp_plan(int L, const LineFFT<float> &f, int top2);
+// largest radix of a plan
+inline int comp_top(const CompFFT &f)
+{
+    int t = 1;
+    for (int s = 0; s < f.ns; s++) t = f.R[s] > t ? f.R[s] : t;
+    return t;
+}
+// Composite-radix passes (comp_x.hip, comp_y.hip, comp_z.hip) for lengths whose
+// prime factors are at most 13; each tells whether it covers the plan's length.
+bool comp_x_applies(const DemagPlanImpl *P);
+bool comp_y_applies(const DemagPlanImpl *P);
+bool comp_z_applies(const DemagPlanImpl *P);    // 3-D
+bool comp_y2d_applies(const DemagPlanImpl *P);  // films
+int comp_xf(const DemagPlanImpl *P, int pred, const float *m, const float *msat_map,
+            const float *tau0, float h, const float *norm_map, float *mpred, hipStream_t st);
+int comp_xi(const DemagPlanImpl *P, int mode, const FieldParams &fp, const EpilogueIO &io,
+            hipStream_t st);
+int comp_yf(const DemagPlanImpl *P, hipStream_t st);
+int comp_yi(const DemagPlanImpl *P, hipStream_t st);
+int comp_z(const DemagPlanImpl *P, hipStream_t st);
+int comp_y2d(const DemagPlanImpl *P, hipStream_t st);
 // The register-FFT x passes run when they have at least this many
 // workgroups (one per CU); below it a handful of workgroups each carry a long
 // serial chain and the generic LDS kernels, spread over more workgroups, are

@@ -357,20 +357,6 @@ template <int L> __device__ __forceinline__ int zrow(int kz)
         return kz;
 }
 
-// ky visiting order 0, p/2, 1, p-1, 2, p-2, ...: tiles of ky and p - ky
-// (which read the same kernel octant rows) are neighbours
-__device__ __forceinline__ int mirror_order(int i, int p)
-{
-    if (i == 0) return 0;
-    if (p & 1) { // odd p: pairs (u, p-u) for u = 1 .. (p-1)/2
-        const int u = (i - 1) / 2 + 1;
-        return (i & 1) ? u : p - u;
-    }
-    if (i == 1) return p / 2;
-    const int u = (i - 2) / 2 + 1;
-    return (i & 1) ? p - u : u;
-}
-
 // FULL: periodic z (n0 == L, every plane holds data); otherwise n0 == L/2
 // and planes n0 .. L-1 are zero padding (not read, not written).  Byte
 // offsets from the wave-uniform bases stay below 4 GiB (fast_z_addressable).

@@ -318,6 +318,20 @@ __device__ __forceinline__ int xcd_tile(int bid, int nb)
     return (x < r) ? x * (q + 1) + l : r * (q + 1) + (x - r) * q + l;
 }
 
+// ky visiting order 0, p/2, 1, p-1, 2, p-2, ...: tiles of ky and p - ky
+// (which read the same kernel octant rows) are neighbours
+__device__ __forceinline__ int mirror_order(int i, int p)
+{
+    if (i == 0) return 0;
+    if (p & 1) { // odd p: pairs (u, p-u) for u = 1 .. (p-1)/2
+        const int u = (i - 1) / 2 + 1;
+        return (i & 1) ? u : p - u;
+    }
+    if (i == 1) return p / 2;
+    const int u = (i - 2) / 2 + 1;
+    return (i & 1) ? p - u : u;
+}
+
 // Forward step 1-2 of the four-step: E-point FFT, then v[k1] *= W_L^(t k1)
 // (twiddle table tw[L] in LDS, forward sign).  HALFIN: the line's upper half
 // (v[E/2 ..]) is zero and not read.

@@ -1,0 +1,81 @@
+"""The composite-radix demag passes at every radix and at the sizes where their
+tiles, stages and plans change: B against a float64 FFT of the plan's own
+real-space kernel."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def mmx():
+    import mmx
+    mmx.check(mmx.lib().mmx_init(0))
+    return mmx
+
+
+def _check(mmx, n, pbc=(0, 0, 0), masked=False):
+    import torch
+    print("comp pass", n, pbc, flush=True)
+    plan = mmx.DemagPlan(n, (3e-9, 4e-9, 4e-9), pbc, keep_real_kernel=True)
+    K = plan.real_kernel().astype(np.float64)
+    K[np.abs(K).max(axis=(1, 2, 3)) < 1e-5 * np.abs(K).max()] = 0.0
+    rng = np.random.default_rng(1000 * n[0] + 10 * n[1] + n[2])
+    m = rng.standard_normal((3,) + n).astype(np.float32)
+    ms = rng.uniform(0.0, 2.0, n).astype(np.float32) if masked else None
+    dm = torch.from_numpy(m).cuda()
+    b = torch.full((3,) + n, np.nan, device="cuda")
+    dms = None if ms is None else torch.from_numpy(ms).cuda()
+    plan.update_b(b.data_ptr(), dm.data_ptr(), 8e5, None if ms is None else dms.data_ptr(), None)
+    torch.cuda.synchronize()
+    S = np.fft.rfftn(m.astype(np.float64) * (1.0 if ms is None else ms), s=plan.p, axes=(1, 2, 3))
+    kh = np.fft.rfftn(K, axes=(1, 2, 3))
+    rows = ((0, 5, 4), (5, 1, 3), (4, 3, 2))
+    F = np.stack([sum(kh[rows[c][s]] * S[s] for s in range(3)) for c in range(3)])
+    want = np.fft.irfftn(F, s=plan.p, axes=(1, 2, 3))[:, :n[0], :n[1], :n[2]] * (4e-7 * np.pi * 8e5)
+    # float32 roundings: some ten per transform, six transforms, and the kernel's own
+    assert np.abs(b.cpu().numpy() - want).max() <= 4e-6 * np.abs(want).max()
+
+
+# x half-lengths: one radix each, two stages of the larger class on many rows,
+# three stages, primes 11 and 13, an odd length
+X = [3, 7, 9, 11, 13, 15, 18, 20, 21, 22, 25, 26, 27, 28, 30, 33, 39, 42, 44, 45, 50, 60, 63, 65, 66, 75, 77, 78, 81,
+     88, 90, 91, 99, 100, 104, 110, 117, 120, 121, 125, 130, 143, 150, 156, 169, 176, 195, 200, 208, 210, 225, 240,
+     250, 270, 286, 300, 343, 360, 375, 420, 500, 600, 625, 729, 1000]
+
+
+@pytest.mark.parametrize("nx", X)
+def test_x_lengths(mmx, nx):
+    _check(mmx, (1, 3, nx))
+
+
+@pytest.mark.parametrize("n,pbc", [((9, 240, 20), (0, 0, 0)), ((1, 6, 100), (0, 0, 1)), ((3, 700, 75), (0, 0, 0)),
+                                   ((1, 5, 1024), (0, 0, 0)), ((2, 10, 130), (0, 0, 1))])
+def test_x_rows(mmx, n, pbc):
+    _check(mmx, n, pbc, masked=True)
+
+
+# y: two and three stages of both classes, columns that do not fill a tile
+@pytest.mark.parametrize("ny", [5, 11, 13, 25, 33, 50, 65, 75, 100, 110, 125, 150, 182, 200, 250, 300, 338, 500, 550,
+                                625, 750, 1000])
+def test_y_lengths(mmx, ny):
+    _check(mmx, (2, ny, 5))
+
+
+@pytest.mark.parametrize("ny,nx,pbc", [(5, 20, 0), (13, 7, 0), (25, 33, 0), (50, 2, 0), (75, 17, 0), (125, 70, 0),
+                                       (100, 9, 1), (200, 40, 0), (250, 3, 0), (300, 16, 0), (500, 5, 0),
+                                       (600, 4, 0), (750, 6, 0), (1000, 9, 0), (1024, 10, 0), (338, 4, 1)])
+def test_film_y_lengths(mmx, ny, nx, pbc):
+    _check(mmx, (1, ny, nx), (0, pbc, 0))
+
+
+# z: every register column length, the lengths behind them, periodic
+@pytest.mark.parametrize("nz", list(range(2, 17)) + [18, 20, 22, 25, 26, 27, 33, 36, 50, 60, 75, 110, 125, 250, 300])
+def test_z_lengths(mmx, nz):
+    _check(mmx, (nz, 4, 9))
+
+
+@pytest.mark.parametrize("n,pbc", [((10, 6, 30), (1, 0, 0)), ((22, 4, 10), (1, 1, 0)), ((5, 70, 50), (0, 1, 0)),
+                                   ((11, 20, 44), (0, 0, 1)), ((36, 10, 40), (0, 0, 0))])
+def test_z_grids(mmx, n, pbc):
+    _check(mmx, n, pbc, masked=True)

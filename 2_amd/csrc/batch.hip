@@ -6,9 +6,12 @@
 //
 //  * one launch per demag pass for all simulations: a block -> simulation
 //    table per pass; each block runs the same tile function as the
-//    single-simulation generic kernels (demag_tiles.hpp), with that
+//    single-simulation composite-radix kernels (comp_tiles.hpp), or the
+//    generic ones (demag_tiles.hpp) for lengths without such a plan, with that
 //    simulation's geometry, FFT plan, buffers and field parameters, read from
-//    a device table;
+//    a device table (32 films of 32x32x1..256x128x4, kernel times of one
+//    evaluation, generic against composite tiles: xf 38 / 22, y 70 / 25, yi 57 /
+//    20, xi 59 / 40 us);
 //  * step control on the device: a one-thread-per-simulation kernel applies
 //    the RK12 controller after every predictor/corrector try and flips the
 //    simulation's m double buffer on acceptance, so no host round trip is
@@ -25,316 +28,47 @@
 #include <cstring>
 #include <vector>
 
-#include "demag_tiles.hpp"
+#include "batch_blocks.hpp"
 #include "sim_impl.hpp"
 
 namespace mmx {
 
-enum BatchPass { BP_XF = 0, BP_Y = 1, BP_Z = 2, BP_YI = 3, BP_XI = 4, BP_N = 5 };
-
-// Per-simulation descriptor, read-only during a launch.
-struct BatchSim {
-    DemagGeom g;
-    LineFFT<float> fx, fy, fz;
-    FieldParams fp;
-    float2 *xbuf, *ybuf;
-    const float *kern;
-    float *mbuf[2];
-    float *mpred, *tau0;
-    const float *msat_map;
-    int zsmall;       // z pass as one thread per column (z_column_small)
-    int tile[BP_N];   // rows (XF, XI) or columns (Y, Z, YI) per workgroup
-    int ntx[BP_N];    // column tiles per line set (Y, Z, YI)
-    int first[BP_N];  // first block of this simulation in each pass
-};
-
-// Per-simulation RK12 state, owned by the device during a run.
-struct BatchState {
-    double t, dt, t0, t_stop, mindt, maxdt, maxerr, err, peakerr, gamma;
-    long long step, step_stop, badsteps, evals;
-    int cur, tries, need_stage0, active, error;
-    float h;
-    unsigned int err_bits;
-    int pad_;
-};
-
-// ------------------------------------------------------------- kernels
-//
-// Each pass is a device function of one virtual block `vb` (a tile of one
-// simulation, from the pass's block table), called by the per-pass kernels
-// with vb = blockIdx.x and by the persistent kernel for vb = blockIdx.x,
-// blockIdx.x + gridDim.x, ...
-
-template <int STAGE>
-__device__ __forceinline__ void bxf_block(const BatchSim *__restrict__ sims,
-                                          const BatchState *__restrict__ st,
-                                          const int *__restrict__ map, int vb, float2 *sm)
+template <int STAGE, int KIND>
+__global__ void __launch_bounds__(kBlock)
+bxf_kernel(const BatchSim *__restrict__ sims, const BatchState *__restrict__ st,
+           const int *__restrict__ map)
 {
-    const int s = map[vb];
-    const BatchSim &S = sims[s];
-    const BatchState &Z = st[s];
-    if (!Z.active || (STAGE == 0 && !Z.need_stage0)) return;
-    const long row0 = (long)(vb - S.first[BP_XF]) * S.tile[BP_XF];
-    const float *m = S.mbuf[Z.cur];
-    if (STAGE == 0)
-        xf_tile<0>(S.g, S.fx, S.tile[BP_XF], row0, m, S.msat_map, nullptr, 0.0f, nullptr, nullptr,
-                   S.xbuf, sm);
-    else
-        xf_tile<1>(S.g, S.fx, S.tile[BP_XF], row0, m, S.msat_map, S.tau0, Z.h, S.msat_map,
-                   S.mpred, S.xbuf, sm);
+    extern __shared__ float2 sm[];
+    bxf_block<STAGE, KIND>(sims, st, map, blockIdx.x, sm);
 }
 
-template <int STAGE>
-__device__ __forceinline__ void by_block(const BatchSim *__restrict__ sims,
-                                         const BatchState *__restrict__ st,
-                                         const int *__restrict__ map, int vb, float2 *sm)
+template <int STAGE, int KIND>
+__global__ void __launch_bounds__(kBlock)
+bxi_kernel(const BatchSim *__restrict__ sims, BatchState *__restrict__ st,
+           const int *__restrict__ map)
 {
-    const int s = map[vb];
-    const BatchSim &S = sims[s];
-    const BatchState &Z = st[s];
-    if (!Z.active || (STAGE == 0 && !Z.need_stage0)) return;
-    const int b = vb - S.first[BP_Y], W = S.tile[BP_Y], ntx = S.ntx[BP_Y];
-    if (S.g.p0 == 1) {
-        y2d_tile(S.g, S.fy, W, b * W, S.kern, S.xbuf, sm);
-    } else {
-        const int kt = b % ntx, i = (b / ntx) % S.g.n0, c = b / (ntx * S.g.n0);
-        yf_tile(S.g, S.fy, W, kt * W, i, c, S.xbuf, S.ybuf, sm);
-    }
+    extern __shared__ float2 sm[];
+    bxi_block<STAGE, KIND>(sims, st, map, blockIdx.x, sm);
 }
 
-template <int STAGE>
-__device__ __forceinline__ void bz_block(const BatchSim *__restrict__ sims,
-                                         const BatchState *__restrict__ st,
-                                         const int *__restrict__ map, int vb, float2 *sm)
-{
-    const int s = map[vb];
-    const BatchSim &S = sims[s];
-    const BatchState &Z = st[s];
-    if (!Z.active || (STAGE == 0 && !Z.need_stage0)) return;
-    const int b = vb - S.first[BP_Z], W = S.tile[BP_Z], ntx = S.ntx[BP_Z];
-    if (S.zsmall) {
-        const long col = (long)b * kBlock + threadIdx.x;
-        if (col >= (long)S.g.p1 * S.g.h2) return;
-        const int ky = (int)(col / S.g.h2), kx = (int)(col - (long)ky * S.g.h2);
-        z_column_small_any(S.g, S.kern, S.ybuf, ky, kx);
-        return;
-    }
-    z_tile(S.g, S.fz, W, (b % ntx) * W, b / ntx, S.kern, S.ybuf, sm);
-}
-
-template <int STAGE>
-__device__ __forceinline__ void byi_block(const BatchSim *__restrict__ sims,
-                                          const BatchState *__restrict__ st,
-                                          const int *__restrict__ map, int vb, float2 *sm)
-{
-    const int s = map[vb];
-    const BatchSim &S = sims[s];
-    const BatchState &Z = st[s];
-    if (!Z.active || (STAGE == 0 && !Z.need_stage0)) return;
-    const int b = vb - S.first[BP_YI], W = S.tile[BP_YI], ntx = S.ntx[BP_YI];
-    const int kt = b % ntx, i = (b / ntx) % S.g.n0, c = b / (ntx * S.g.n0);
-    yi_tile(S.g, S.fy, W, kt * W, i, c, S.ybuf, S.xbuf, sm);
-}
-
-// STAGE 0: tau0 = torque(m) (solve_rk12.go:97-115); STAGE 1: corrector,
-// normalised m into the other buffer, max |tau1 - tau0| into err_bits.
-template <int STAGE>
-__device__ __forceinline__ void bxi_block(const BatchSim *__restrict__ sims,
-                                          BatchState *__restrict__ st,
-                                          const int *__restrict__ map, int vb, float2 *sm)
-{
-    const int s = map[vb];
-    const BatchSim &S = sims[s];
-    BatchState &Z = st[s];
-    if (!Z.active || (STAGE == 0 && !Z.need_stage0)) return;
-    const long row0 = (long)(vb - S.first[BP_XI]) * S.tile[BP_XI];
-    EpilogueIO io{};
-    if (STAGE == 0) {
-        io.m = S.mbuf[Z.cur];
-        io.tout = S.tau0;
-        xi_tile<EPI_TAU0>(S.g, S.fx, S.tile[BP_XI], row0, S.xbuf, S.fp, io, sm);
-    } else {
-        io.m = S.mpred;
-        io.tau0 = S.tau0;
-        io.mnew = S.mbuf[Z.cur ^ 1];
-        io.h = Z.h;
-        io.err = &Z.err_bits;
-        xi_tile<EPI_CORR>(S.g, S.fx, S.tile[BP_XI], row0, S.xbuf, S.fp, io, sm);
-    }
-}
-
-#define MMX_BATCH_KERNEL(NAME, BODY, STATE_T)                                                \
-    template <int STAGE>                                                                     \
+#define MMX_BATCH_KERNEL(NAME, BODY)                                                         \
+    template <int KIND>                                                                      \
     __global__ void __launch_bounds__(kBlock)                                                \
-    NAME(const BatchSim *__restrict__ sims, STATE_T *__restrict__ st,                        \
+    NAME(int stage, const BatchSim *__restrict__ sims, const BatchState *__restrict__ st,    \
          const int *__restrict__ map)                                                        \
     {                                                                                        \
         extern __shared__ float2 sm[];                                                       \
-        BODY<STAGE>(sims, st, map, blockIdx.x, sm);                                          \
+        BODY<KIND>(stage, sims, st, map, blockIdx.x, sm);                                          \
     }
-MMX_BATCH_KERNEL(bxf_kernel, bxf_block, const BatchState)
-MMX_BATCH_KERNEL(by_kernel, by_block, const BatchState)
-MMX_BATCH_KERNEL(bz_kernel, bz_block, const BatchState)
-MMX_BATCH_KERNEL(byi_kernel, byi_block, const BatchState)
-MMX_BATCH_KERNEL(bxi_kernel, bxi_block, BatchState)
+MMX_BATCH_KERNEL(by_kernel, by_block)
+MMX_BATCH_KERNEL(bz_kernel, bz_block)
+MMX_BATCH_KERNEL(byi_kernel, byi_block)
 #undef MMX_BATCH_KERNEL
-
-// RK12Solver.Step's controller (solve_rk12.go:124-214) after one try, for one
-// simulation; mirrors the host loop of mmx_sim_step.
-__device__ __forceinline__ void control_one(BatchState &Z)
-{
-    if (!Z.active) return;
-    const int maxTry = 10;
-    const double headRoom = 0.8;
-    const float maxdiff = __uint_as_float(Z.err_bits);
-    Z.err_bits = 0u;
-    Z.evals += Z.need_stage0 ? 2 : 1;
-    if (!isfinite(maxdiff)) {
-        Z.error = MMX_ERR_NAN;
-        Z.active = 0;
-        return;
-    }
-    const float stepDiff = maxdiff * Z.h;
-    const double err = (double)stepDiff;
-    const double dt = Z.dt;
-    Z.t = Z.t0 + dt;
-    Z.err = err;
-    bool bad = false;
-    if (err > Z.maxerr) {
-        Z.badsteps++;
-        bad = true;
-    }
-    if ((!bad || Z.tries == maxTry - 1) && err > Z.peakerr) Z.peakerr = err;
-    double factor = bad ? pow(Z.maxerr / err, 1.0 / 3.0) : sqrt(Z.maxerr / err);
-    factor *= headRoom;
-    if (factor > 1.5) factor = 1.5;
-    if (factor < 0.1) factor = 0.1;
-    const double minFactor = factor < 2.0 ? factor : 2.0;
-    double newDt = dt * minFactor;
-    if (newDt < Z.mindt) newDt = Z.mindt;
-    if (newDt > Z.maxdt) newDt = Z.maxdt;
-    Z.dt = newDt;
-    if (!bad || newDt == Z.mindt) {
-        Z.cur ^= 1;
-        Z.step++;
-        Z.tries = 0;
-        Z.need_stage0 = 1;
-        Z.t0 = Z.t;
-        if (Z.t >= Z.t_stop || Z.step >= Z.step_stop) Z.active = 0;
-    } else {
-        if (Z.tries > maxTry) {
-            Z.error = MMX_ERR_CONVERGE;
-            Z.active = 0;
-            return;
-        }
-        Z.tries++;
-        Z.need_stage0 = 0;
-    }
-    Z.h = (float)(Z.dt * Z.gamma);
-}
 
 __global__ void __launch_bounds__(64) bcontrol_kernel(BatchState *__restrict__ st, int nsim)
 {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
     if (s < nsim) control_one(st[s]);
-}
-
-// ---------------------------------------------------- the persistent launch
-//
-// One cooperative launch (every workgroup resident) runs up to `tries` tries
-// of the whole batch: the ten passes of a try and the controller one after
-// another, separated by grid-wide barriers, each pass's virtual blocks dealt
-// round-robin to the workgroups.  It stops early once no simulation is
-// active.  A barrier wait is bounded: past kSpinLimit polls the workgroup
-// records the time-out in `fail` and leaves; a timed-out barrier leaves the
-// barrier words inconsistent, so the host resets them before the next launch.
-
-struct PersistArgs {
-    const int *map[BP_N];
-    int nblk[BP_N];
-    int nsim;
-    int tries;
-    unsigned int *bar;   // [0]: arrivals, [1]: generation
-    unsigned int *fail;  // nonzero: a barrier wait timed out
-    int *nactive;        // active simulations after the last controller run
-};
-
-constexpr long kSpinLimit = 1L << 25;
-
-// Grid-wide barrier with agent-scope release/acquire (the workgroups of the
-// 8 XCDs do not share an L2).  Returns false when the wait timed out.
-__device__ bool grid_barrier(const PersistArgs &a)
-{
-    __shared__ int ok;
-    __threadfence();
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        const unsigned int gen =
-            __hip_atomic_load(&a.bar[1], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT);
-        const unsigned int arrived =
-            __hip_atomic_fetch_add(&a.bar[0], 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
-        ok = 1;
-        if (arrived == gridDim.x - 1) {
-            __hip_atomic_store(&a.bar[0], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_fetch_add(&a.bar[1], 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-        } else {
-            long n = 0;
-            while (__hip_atomic_load(&a.bar[1], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT) ==
-                   gen) {
-                __builtin_amdgcn_s_sleep(2);
-                if (++n > kSpinLimit) {
-                    __hip_atomic_store(a.fail, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    ok = 0;
-                    break;
-                }
-            }
-        }
-    }
-    __syncthreads();
-    __threadfence();
-    return ok != 0;
-}
-
-template <int STAGE>
-__device__ bool persist_passes(const BatchSim *__restrict__ sims, BatchState *__restrict__ st,
-                               const PersistArgs &a, float2 *sm)
-{
-#define MMX_PASS(P, BODY)                                                                    \
-    if (a.nblk[P] > 0) {                                                                     \
-        for (int vb = blockIdx.x; vb < a.nblk[P]; vb += gridDim.x) {                         \
-            BODY<STAGE>(sims, st, a.map[P], vb, sm);                                         \
-            __syncthreads(); /* the next tile reuses the LDS */                              \
-        }                                                                                    \
-        if (!grid_barrier(a)) return false;                                                  \
-    }
-    MMX_PASS(BP_XF, bxf_block)
-    MMX_PASS(BP_Y, by_block)
-    MMX_PASS(BP_Z, bz_block)
-    MMX_PASS(BP_YI, byi_block)
-    MMX_PASS(BP_XI, bxi_block)
-#undef MMX_PASS
-    return true;
-}
-
-__global__ void __launch_bounds__(kBlock)
-bpersist_kernel(const BatchSim *__restrict__ sims, BatchState *__restrict__ st, PersistArgs a)
-{
-    extern __shared__ float2 sm[];
-    for (int k = 0; k < a.tries; k++) {
-        if (!persist_passes<0>(sims, st, a, sm)) return;
-        if (!persist_passes<1>(sims, st, a, sm)) return;
-        if (blockIdx.x == 0) {
-            for (int s = threadIdx.x; s < a.nsim; s += blockDim.x) control_one(st[s]);
-            __syncthreads();
-            if (threadIdx.x == 0) {
-                int n = 0;
-                for (int s = 0; s < a.nsim; s++) n += st[s].active;
-                __hip_atomic_store(a.nactive, n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            }
-        }
-        if (!grid_barrier(a)) return;
-        if (__hip_atomic_load(a.nactive, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0) return;
-    }
 }
 
 // ------------------------------------------------------------ host side
@@ -348,6 +82,7 @@ struct BatchImpl {
     int *dmap[BP_N] = {};
     int nblk[BP_N] = {};
     size_t lds[BP_N] = {};
+    int kind[BP_N] = {};        // BatchKind of each pass's kernel
     size_t cap[BP_N] = {};      // LDS budget per pass (tuner's choice)
     hipStream_t st = nullptr;
     hipGraphExec_t gexec = nullptr;
@@ -368,9 +103,31 @@ struct mmx_batch {
 namespace mmx {
 namespace {
 
-// LDS bytes a pass needs for tile parameter v of simulation g
-size_t pass_lds(int pass, const DemagGeom &g, int v)
+bool comp_pass(int pass, const BatchSim &S)
 {
+    switch (pass) {
+    case BP_XF:
+    case BP_XI: return S.cx.ns > 0;
+    case BP_Z: return S.cz.ns > 0;
+    default: return S.cy.ns > 0;
+    }
+}
+
+// LDS bytes a pass needs for tile parameter v (rows, or columns: a power of two
+// on the composite passes) of simulation S
+size_t pass_lds(int pass, const BatchSim &S, int v)
+{
+    const DemagGeom &g = S.g;
+    if (comp_pass(pass, S)) {
+        const int lw = __builtin_ctz(v);
+        switch (pass) {
+        case BP_XF:
+        case BP_XI: return comp_x_lds(S.cx, v);
+        case BP_Y: return g.p0 == 1 ? comp_z_lds(S.cy, lw) : comp_y_lds(S.cy, lw);
+        case BP_Z: return comp_z_lds(S.cz, lw);
+        default: return comp_y_lds(S.cy, lw);
+        }
+    }
     switch (pass) {
     case BP_XF:
     case BP_XI: return 2ull * 3 * v * (g.Lx + 1) * sizeof(float2);
@@ -386,10 +143,11 @@ bool pass_applies(int pass, const DemagGeom &g)
 }
 
 // largest tile parameter (<= 16) whose LDS fits the budget, at least 1
-int pick_tile(int pass, const DemagGeom &g, size_t budget)
+int pick_tile(int pass, const BatchSim &S, size_t budget)
 {
+    const bool pow2 = comp_pass(pass, S) && pass != BP_XF && pass != BP_XI;
     int v = 16;
-    while (v > 1 && pass_lds(pass, g, v) > budget) v--;
+    while (v > 1 && pass_lds(pass, S, v) > budget) v = pow2 ? v / 2 : v - 1;
     return v;
 }
 
@@ -417,18 +175,30 @@ template <typename K> void allow_lds_batch(K kernel, size_t bytes)
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
 }
 
+// f(kind) for the pass's kind as a constant
+template <typename F> void with_kind(const BatchImpl &B, int p, F f)
+{
+    if (B.kind[p] == KIND_ANY)
+        f(std::integral_constant<int, KIND_ANY>{});
+    else if (B.kind[p] == KIND_ZCOL)
+        f(std::integral_constant<int, KIND_ZCOL>{});
+    else
+        f(std::integral_constant<int, KIND_COMP>{});
+}
+
 void set_attributes(const BatchImpl &B)
 {
-    allow_lds_batch(bxf_kernel<0>, B.lds[BP_XF]);
-    allow_lds_batch(bxf_kernel<1>, B.lds[BP_XF]);
-    allow_lds_batch(by_kernel<0>, B.lds[BP_Y]);
-    allow_lds_batch(by_kernel<1>, B.lds[BP_Y]);
-    allow_lds_batch(bz_kernel<0>, B.lds[BP_Z]);
-    allow_lds_batch(bz_kernel<1>, B.lds[BP_Z]);
-    allow_lds_batch(byi_kernel<0>, B.lds[BP_YI]);
-    allow_lds_batch(byi_kernel<1>, B.lds[BP_YI]);
-    allow_lds_batch(bxi_kernel<0>, B.lds[BP_XI]);
-    allow_lds_batch(bxi_kernel<1>, B.lds[BP_XI]);
+    with_kind(B, BP_XF, [&](auto K) {
+        allow_lds_batch(bxf_kernel<0, K.value>, B.lds[BP_XF]);
+        allow_lds_batch(bxf_kernel<1, K.value>, B.lds[BP_XF]);
+    });
+    with_kind(B, BP_Y, [&](auto K) { allow_lds_batch(by_kernel<K.value>, B.lds[BP_Y]); });
+    with_kind(B, BP_Z, [&](auto K) { allow_lds_batch(bz_kernel<K.value>, B.lds[BP_Z]); });
+    with_kind(B, BP_YI, [&](auto K) { allow_lds_batch(byi_kernel<K.value>, B.lds[BP_YI]); });
+    with_kind(B, BP_XI, [&](auto K) {
+        allow_lds_batch(bxi_kernel<0, K.value>, B.lds[BP_XI]);
+        allow_lds_batch(bxi_kernel<1, K.value>, B.lds[BP_XI]);
+    });
 }
 
 void drop_graph(BatchImpl &B)
@@ -447,26 +217,30 @@ int build_tables(BatchImpl &B)
     std::vector<int> maps[BP_N];
     for (int p = 0; p < BP_N; p++) {
         B.lds[p] = 0;
+        bool any = false, comp = false;
         for (int s = 0; s < ns; s++) {
             BatchSim &S = B.hs[s];
             S.first[p] = (int)maps[p].size();
             S.tile[p] = 1;
             S.ntx[p] = 0;
             if (!pass_applies(p, S.g)) continue;
-            if (p == BP_Z && S.zsmall) {
-                const int nb = (int)div_up((long)S.g.p1 * S.g.h2, kBlock);
+            if (p == BP_Z && S.zcol) {
+                const int nb = (int)div_up((long)S.g.p1 * S.g.h2, kZCols);
                 maps[p].insert(maps[p].end(), (size_t)nb, s);
+                B.lds[p] = std::max(B.lds[p], zcol_lds(S.g.n0));
                 continue;
             }
-            const int v = pick_tile(p, S.g, B.cap[p]);
+            (comp_pass(p, S) ? comp : any) = true;
+            const int v = pick_tile(p, S, B.cap[p]);
             S.tile[p] = v;
             const int nb = pass_blocks(p, S.g, v, &S.ntx[p]);
             maps[p].insert(maps[p].end(), (size_t)nb, s);
-            B.lds[p] = std::max(B.lds[p], pass_lds(p, S.g, v));
+            B.lds[p] = std::max(B.lds[p], pass_lds(p, S, v));
         }
         MMX_REQUIRE(B.lds[p] <= 160 * 1024, MMX_ERR_SIZE,
                     "batch: pass %d needs %zu bytes of LDS per workgroup", p, B.lds[p]);
         B.nblk[p] = (int)maps[p].size();
+        B.kind[p] = any ? KIND_ANY : (p == BP_Z && !comp) ? KIND_ZCOL : KIND_COMP;
         (void)hipFree(B.dmap[p]);
         B.dmap[p] = nullptr;
         if (B.nblk[p] > 0) {
@@ -479,6 +253,17 @@ int build_tables(BatchImpl &B)
     drop_graph(B);
     B.tables_dirty = false;
     return MMX_OK;
+}
+
+// (the radices are searched once: the lengths of a simulation stay)
+void batch_plan(CompFFT &c, int L, const LineFFT<float> &f)
+{
+    if (c.L != L) {
+        c = comp_plan(L, f, 16);
+        if (comp_top(c) > 16) c.ns = 0;
+    }
+    c.tw = f.tw;
+    c.rtw = f.rtw;
 }
 
 // Descriptor and state of every simulation from its current host settings.
@@ -510,7 +295,15 @@ int load_sims(BatchImpl &B, double duration, long long nsteps)
         S.mpred = x->mpred;
         S.tau0 = x->tau0;
         S.msat_map = x->msat_map;
-        S.zsmall = z_small_applies(P.g) ? 1 : 0;
+        // the composite passes in their small class (registers for four waves per
+        // SIMD): lengths without radices up to 16 take the generic tiles
+        batch_plan(S.cx, P.g.Lx, P.fx);
+        batch_plan(S.cy, P.g.p1, P.fy);
+        batch_plan(S.cz, P.g.p0, P.fz);
+        S.zcol = (2 * P.g.n0 == P.g.p0 && P.g.n0 >= 2 && P.g.n0 <= 8 &&
+                  (double)P.g.p1 * P.g.h2 + kZCols < 2147483647.0)
+                     ? 1
+                     : 0;
         BatchState &Z = B.hst[s];
         std::memset(&Z, 0, sizeof(Z));
         Z.t = Z.t0 = x->t;
@@ -547,14 +340,34 @@ void launch(K kernel, int nblk, size_t lds, hipStream_t st, const BatchSim *sims
 }
 
 // one evaluation of stage STAGE over the batch: the five passes
+template <typename K>
+void launch_stage(K kernel, int stage, int nblk, size_t lds, hipStream_t st, const BatchSim *sims,
+                  const BatchState *bst, const int *map)
+{
+    if (nblk > 0) kernel<<<dim3(nblk), dim3(kBlock), lds, st>>>(stage, sims, bst, map);
+}
+
 template <int STAGE> int eval_passes(BatchImpl &B, int only_pass = -1)
 {
     auto want = [&](int p) { return only_pass < 0 || only_pass == p; };
-    if (want(BP_XF)) launch(bxf_kernel<STAGE>, B.nblk[BP_XF], B.lds[BP_XF], B.st, B.dsims, B.dst, B.dmap[BP_XF]);
-    if (want(BP_Y)) launch(by_kernel<STAGE>, B.nblk[BP_Y], B.lds[BP_Y], B.st, B.dsims, B.dst, B.dmap[BP_Y]);
-    if (want(BP_Z)) launch(bz_kernel<STAGE>, B.nblk[BP_Z], B.lds[BP_Z], B.st, B.dsims, B.dst, B.dmap[BP_Z]);
-    if (want(BP_YI)) launch(byi_kernel<STAGE>, B.nblk[BP_YI], B.lds[BP_YI], B.st, B.dsims, B.dst, B.dmap[BP_YI]);
-    if (want(BP_XI)) launch(bxi_kernel<STAGE>, B.nblk[BP_XI], B.lds[BP_XI], B.st, B.dsims, B.dst, B.dmap[BP_XI]);
+#define MMX_LAUNCH(P, KERNEL)                                                                \
+    if (want(P))                                                                             \
+        with_kind(B, P, [&](auto K) {                                                        \
+            launch(KERNEL, B.nblk[P], B.lds[P], B.st, B.dsims, B.dst, B.dmap[P]);            \
+        });
+#define MMX_LAUNCH_STAGE(P, KERNEL)                                                          \
+    if (want(P))                                                                             \
+        with_kind(B, P, [&](auto K) {                                                        \
+            launch_stage(KERNEL, STAGE, B.nblk[P], B.lds[P], B.st, B.dsims, B.dst,           \
+                         B.dmap[P]);                                                         \
+        });
+    MMX_LAUNCH(BP_XF, (bxf_kernel<STAGE, K.value>))
+    MMX_LAUNCH_STAGE(BP_Y, by_kernel<K.value>)
+    MMX_LAUNCH_STAGE(BP_Z, bz_kernel<K.value>)
+    MMX_LAUNCH_STAGE(BP_YI, byi_kernel<K.value>)
+    MMX_LAUNCH(BP_XI, (bxi_kernel<STAGE, K.value>))
+#undef MMX_LAUNCH
+#undef MMX_LAUNCH_STAGE
     if (hipGetLastError() != hipSuccess) {
         set_error("batch pass launch failed");
         return MMX_ERR_HIP;
@@ -614,13 +427,14 @@ int persist_launch(BatchImpl &B)
     a.bar = B.dpersist;
     a.fail = B.dpersist + 2;
     a.nactive = reinterpret_cast<int *>(B.dpersist + 3);
-    allow_lds_batch(bpersist_kernel, lds);
+    const void *kernel = persist_kernel();
+    MMX_HIP(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     int dev = 0, coop = 0, ncu = 0, per_cu = 0;
     MMX_HIP(hipGetDevice(&dev));
     MMX_HIP(hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev));
     MMX_REQUIRE(coop, MMX_ERR_STATE, "batch: the device has no cooperative launch");
     MMX_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
-    MMX_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, bpersist_kernel, kBlock, lds));
+    MMX_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kBlock, lds));
     MMX_REQUIRE(per_cu > 0, MMX_ERR_SIZE, "batch: the persistent kernel does not fit a CU (%zu B LDS)",
                 lds);
     const int grid = std::max(1, std::min(per_cu * ncu, maxblk));
@@ -630,8 +444,7 @@ int persist_launch(BatchImpl &B)
     const BatchSim *sims = B.dsims;
     BatchState *st = B.dst;
     void *args[] = {&sims, &st, &a};
-    MMX_HIP(hipLaunchCooperativeKernel(reinterpret_cast<const void *>(bpersist_kernel),
-                                       dim3(grid), dim3(kBlock), args, (unsigned int)lds, B.st));
+    MMX_HIP(hipLaunchCooperativeKernel(kernel, dim3(grid), dim3(kBlock), args, (unsigned int)lds, B.st));
     unsigned int h[4];
     MMX_HIP(hipMemcpyAsync(h, B.dpersist, sizeof(h), hipMemcpyDeviceToHost, B.st));
     MMX_HIP(hipStreamSynchronize(B.st));

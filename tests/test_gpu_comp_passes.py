@@ -79,3 +79,30 @@ def test_z_lengths(mmx, nz):
                                    ((11, 20, 44), (0, 0, 1)), ((36, 10, 40), (0, 0, 0))])
 def test_z_grids(mmx, n, pbc):
     _check(mmx, n, pbc, masked=True)
+
+
+# batches whose passes hold the composite tiles alone, the 64-column z tile
+# alone, and generic tiles next to them (primes above 13, a radix above 16)
+BATCHES = [[(1, 16, 32), (1, 20, 50)], [(2, 16, 32), (4, 12, 20), (8, 6, 10)], [(9, 8, 16), (2, 16, 32), (1, 30, 21)],
+           [(1, 17, 19), (2, 16, 32), (3, 34, 10)], [(1, 250, 4), (20, 4, 6), (1, 625, 2)]]
+
+
+@pytest.mark.parametrize("grids", BATCHES)
+def test_batch_tiles(mmx, grids):
+    def make(n, k):
+        s = mmx.Sim(n, (3e-9, 4e-9, 4e-9))
+        for name, v in (("Msat", 8e5), ("Aex", 1.3e-11), ("alpha", 0.1), ("m_maxerror", 1e-5), ("dt", 1e-14)):
+            s.setv(name, v)
+        s.load("zhang-li")
+        s.setv("j", (0.0, 0.0, 1e12))
+        s.setarray("m", np.random.default_rng(k).standard_normal((3,) + n).astype(np.float32))
+        return s
+    print("batch", grids, flush=True)
+    one = [make(n, k) for k, n in enumerate(grids)]
+    both = [make(n, k) for k, n in enumerate(grids)]
+    mmx.Batch(both).steps(3)
+    for a, b in zip(one, both):
+        a.steps(3)
+        # three steps of float32 stages of the same arithmetic in other transforms
+        assert np.abs(a.getarray("m") - b.getarray("m")).max() < 5e-6
+        assert a.getv("step") == b.getv("step") == 3

@@ -300,6 +300,11 @@ int load_sims(BatchImpl &B, double duration, long long nsteps)
         batch_plan(S.cx, P.g.Lx, P.fx);
         batch_plan(S.cy, P.g.p1, P.fy);
         batch_plan(S.cz, P.g.p0, P.fz);
+        const DemagGeom &g = P.g;
+        const long es = (long)g.p1 * g.sx;
+        if (!comp_x_fits(g)) S.cx.ns = 0;
+        if (S.cz.ns && !comp_line_fits(g.n0 * es, es, S.cz.L / S.cz.R[0])) S.cz.ns = 0;
+        if (S.cy.ns && g.p0 == 1 && !comp_line_fits(g.nrows * g.sx, g.sx, S.cy.L / S.cy.R[0])) S.cy.ns = 0;
         S.zcol = (2 * P.g.n0 == P.g.p0 && P.g.n0 >= 2 && P.g.n0 <= 8 &&
                   (double)P.g.p1 * P.g.h2 + kZCols < 2147483647.0)
                      ? 1

@@ -195,6 +195,7 @@ __device__ __forceinline__ void bxi_block(const BatchSim *__restrict__ sims,
         io.mnew = S.mbuf[Z.cur ^ 1];
         io.h = Z.h;
         io.err = &Z.err_bits;
+        io.err_mask = 0;
         if (KIND != KIND_ANY || S.cx.ns)
             xi_comp_tile<16, EPI_CORR>(S.g, S.cx, S.tile[BP_XI], row0, S.xbuf, S.fp, io, sm);
         else

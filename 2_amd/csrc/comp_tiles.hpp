@@ -6,7 +6,7 @@
 #pragma once
 
 #include "comp_fft.hpp"
-#include "epilogue.hpp"
+#include "pair_epilogue.hpp"
 
 namespace mmx {
 
@@ -17,6 +17,13 @@ __device__ __forceinline__ void load_tw(const CompFFT &f, float2 *stw)
 }
 
 // ------------------------------------------------------------------ x passes
+
+// The x passes address cells and spectrum rows with 32-bit byte offsets.
+__host__ __device__ inline bool comp_x_fits(const DemagGeom &g)
+{
+    return g.N < kMaxCells32 && ((double)g.nrows + 16) * g.sx * sizeof(float2) < 4294967295.0 &&
+           (g.n2 == g.Lx || g.n2 == 2 * g.Lx);
+}
 
 // LDS (bytes): 3 RB lines, twiddles
 __host__ __device__ inline size_t comp_x_lds(const CompFFT &f, int RB)
@@ -44,7 +51,7 @@ __device__ __forceinline__ void
 xf_comp_tile(const DemagGeom &g, const CompFFT &f, int RB, long row0, const float *__restrict__ m,
              const float *__restrict__ msat_map, const float *__restrict__ tau0, float h,
              const float *__restrict__ norm_map, float *__restrict__ mpred,
-             float2 *__restrict__ xb, float2 *sm)
+             float2 *__restrict__ xb, float2 *sm, bool pairs = false)
 {
     const int L = f.L;
     const RowLines ln{3 * RB, comp_slots(f)};
@@ -55,40 +62,46 @@ xf_comp_tile(const DemagGeom &g, const CompFFT &f, int RB, long row0, const floa
         const int r = f.byL.quot(t), e = t - r * L;
         const long row = row0 + r;
         float v[2][3] = {{0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f}};
-        if (row < g.nrows) {
+        if (row < g.nrows && 2 * e < g.n2) {
+            const unsigned I = 4u * (unsigned)((int)row * g.n2 + 2 * e); // byte offset
+            const bool two = 2 * e + 1 < g.n2;
+            // the cell pair of a component array; one cell at the end of an odd
+            // row, and two loads where the array is not 8-byte aligned
+            auto ld2 = [&](const float *p) {
+                return pairs ? ld_off<float2>(p, I)
+                             : float2{ld_off<float>(p, I), two ? ld_off<float>(p, I + 4u) : 0.0f};
+            };
+            float2 x[3] = {ld2(m), ld2(m + N), ld2(m + 2 * N)};
+            if (PRED) {
+                // predictor m = y0 + dt*gamma*tau0 (maddKern), then the
+                // normUpdater (normalize.cu:14-43)
+                const float2 t0[3] = {ld2(tau0), ld2(tau0 + N), ld2(tau0 + 2 * N)};
+                const float2 nm = norm_map ? ld2(norm_map) : float2{1.0f, 1.0f};
 #pragma unroll
-            for (int q = 0; q < 2; q++) {
-                const int k = 2 * e + q;
-                if (k < g.n2) {
-                    const long I = row * g.n2 + k;
-                    float a0 = m[I], a1 = m[N + I], a2 = m[2 * N + I];
-                    if (PRED) {
-                        // predictor m = y0 + dt*gamma*tau0 (maddKern), then the
-                        // normUpdater (normalize.cu:14-43)
-                        a0 = a0 + h * tau0[I];
-                        a1 = a1 + h * tau0[N + I];
-                        a2 = a2 + h * tau0[2 * N + I];
-                        const float norm = norm_map ? norm_map[I] : 1.0f;
-                        const float len = sqrtf(a0 * a0 + a1 * a1 + a2 * a2);
-                        float scale = (norm == 0.0f) ? 0.0f : 1.0f;
-                        scale = (len != 0.0f) ? scale / len : 0.0f;
-                        a0 *= scale;
-                        a1 *= scale;
-                        a2 *= scale;
-                        mpred[I] = a0;
-                        mpred[N + I] = a1;
-                        mpred[2 * N + I] = a2;
+                for (int c = 0; c < 3; c++) x[c] = float2{x[c].x + h * t0[c].x, x[c].y + h * t0[c].y};
+                auto unit = [](float a, float b, float c, float norm) {
+                    const float len = sqrtf(a * a + b * b + c * c);
+                    const float scale = (norm == 0.0f) ? 0.0f : 1.0f;
+                    return (len != 0.0f) ? scale / len : 0.0f;
+                };
+                const float s0 = unit(x[0].x, x[1].x, x[2].x, nm.x);
+                const float s1 = unit(x[0].y, x[1].y, x[2].y, nm.y);
+#pragma unroll
+                for (int c = 0; c < 3; c++) {
+                    x[c] = float2{x[c].x * s0, x[c].y * s1};
+                    if (pairs) {
+                        st_off<float2>(mpred + c * N, I, x[c]);
+                    } else {
+                        st_off<float>(mpred + c * N, I, x[c].x);
+                        if (two) st_off<float>(mpred + c * N, I + 4u, x[c].y);
                     }
-                    if (msat_map) {
-                        const float ms = msat_map[I];
-                        a0 *= ms;
-                        a1 *= ms;
-                        a2 *= ms;
-                    }
-                    v[q][0] = a0;
-                    v[q][1] = a1;
-                    v[q][2] = a2;
                 }
+            }
+            const float2 ms = msat_map ? ld2(msat_map) : float2{1.0f, 1.0f};
+#pragma unroll
+            for (int c = 0; c < 3; c++) {
+                v[0][c] = msat_map ? x[c].x * ms.x : x[c].x;
+                v[1][c] = two ? (msat_map ? x[c].y * ms.y : x[c].y) : 0.0f;
             }
         }
 #pragma unroll
@@ -104,21 +117,26 @@ xf_comp_tile(const DemagGeom &g, const CompFFT &f, int RB, long row0, const floa
         if (row >= g.nrows) continue;
         const float2 w = f.rtw[k];
         const int pa = slot_out(f, k), pb = slot_out(f, k == 0 ? 0 : L - k);
+        const unsigned o = 8u * ((unsigned)row * (unsigned)g.sx + (unsigned)k);
 #pragma unroll
         for (int c = 0; c < 3; c++) {
             const float2 a = A[ln.at(c * RB + r, pa)];
             const float2 b = cconj(A[ln.at(c * RB + r, pb)]);
             const float2 E = float2{0.5f * (a.x + b.x), 0.5f * (a.y + b.y)};
             const float2 O = float2{0.5f * (a.y - b.y), -0.5f * (a.x - b.x)};
-            float2 *dst = xb + ((long)c * g.nrows + row) * g.sx;
-            dst[k] = cadd(E, cmul(O, w));
+            float2 *dst = xb + (long)c * g.nrows * g.sx;
+            st_off<float2>(dst, o, cadd(E, cmul(O, w)));
             // the last bin, E(0) - O(0)
-            if (k == 0) dst[L] = float2{a.x - a.y, 0.0f};
+            if (k == 0) st_off<float2>(dst, o + 8u * (unsigned)L, float2{a.x - a.y, 0.0f});
         }
     }
 }
 
-template <int RM, int MODE>
+// PAIR 0: one cell at a time, every term; 1, 2: two cells at a time with 8-byte
+// accesses, uniform parameters or maps, no spin-transfer term, n2 even
+// (pair_epilogue) -- for grids with enough rows that the epilogue's
+// instructions, not its latency, take the time
+template <int RM, int MODE, int PAIR = 0>
 __device__ __forceinline__ void
 xi_comp_tile(const DemagGeom &g, const CompFFT &f, int RB, long row0,
              const float2 *__restrict__ xb, const FieldParams &fp, const EpilogueIO &io, float2 *sm)
@@ -141,20 +159,23 @@ xi_comp_tile(const DemagGeom &g, const CompFFT &f, int RB, long row0,
     // together with the spectrum (their latency would follow the transform's)
     CellLocal loc;
     int r, k, i, j;
-    const bool have = (int)threadIdx.x < RB * g.n2 && place(threadIdx.x, r, k, i, j);
-    if (have) cell_local<MODE>(g, fp, io, (row0 + r) * g.n2 + k, i, j, k, loc);
+    const bool have = PAIR == 0 && (int)threadIdx.x < RB * g.n2 && place(threadIdx.x, r, k, i, j);
+    if (have)
+        cell_local<MODE, unsigned>(g, fp, io, (unsigned)(((int)row0 + r) * g.n2 + k), i, j, k, loc);
     // C2R pre-processing (imaginary parts of DC and Nyquist ignored)
     for (int t = threadIdx.x; t < RB * L; t += kBlock) {
         const int r = f.byL.quot(t), k = t - r * L;
         const long row = row0 + r;
         const float2 w = f.rtw[k];
         const int p = slot_in(f, k);
+        const unsigned o = 8u * (unsigned)row * (unsigned)g.sx;
 #pragma unroll
         for (int c = 0; c < 3; c++) {
             float2 z = float2{0.0f, 0.0f};
             if (row < g.nrows) {
-                const float2 *src = xb + ((long)c * g.nrows + row) * g.sx;
-                float2 a = src[k], bb = src[L - k];
+                const float2 *src = xb + (long)c * g.nrows * g.sx;
+                float2 a = ld_off<float2>(src, o + 8u * (unsigned)k),
+                       bb = ld_off<float2>(src, o + 8u * (unsigned)(L - k));
                 if (k == 0) {
                     a.y = 0.0f;
                     bb.y = 0.0f;
@@ -171,11 +192,28 @@ xi_comp_tile(const DemagGeom &g, const CompFFT &f, int RB, long row0,
     row_lines_fft<RM, +1>(f, ln, A, stw);
 
     float errmax = 0.0f;
+    if constexpr (PAIR > 0) {
+        for (int t = threadIdx.x; t < RB * g.n2 / 2; t += kBlock) {
+            if (!place(2 * t, r, k, i, j)) continue;
+            float hd0[3], hd1[3];
+            const int p = slot_out(f, k >> 1);
+#pragma unroll
+            for (int c = 0; c < 3; c++) {
+                const float2 z = A[ln.at(c * RB + r, p)];
+                hd0[c] = fp.demag_scale * z.x;
+                hd1[c] = fp.demag_scale * z.y;
+            }
+            pair_epilogue<MODE, PAIR == 2>(g, fp, io, (unsigned)(((int)row0 + r) * g.n2 + k), i, j, k, hd0,
+                                           hd1, errmax);
+        }
+        if (MODE == EPI_CORR) block_max_slot(errmax, io.err, io.err_mask);
+        return;
+    }
     for (int t = threadIdx.x; t < RB * g.n2; t += kBlock) {
         const bool ok = place(t, r, k, i, j);
         if (!ok) continue;
         const long I = (row0 + r) * g.n2 + k;
-        if (t >= kBlock) cell_local<MODE>(g, fp, io, I, i, j, k, loc);
+        if (t >= kBlock) cell_local<MODE, unsigned>(g, fp, io, (unsigned)I, i, j, k, loc);
         float hd[3];
         const int p = slot_out(f, k >> 1);
 #pragma unroll
@@ -185,7 +223,7 @@ xi_comp_tile(const DemagGeom &g, const CompFFT &f, int RB, long row0,
         }
         cell_finish<MODE>(g, fp, io, I, loc, hd, errmax);
     }
-    if (MODE == EPI_CORR) block_max_to(errmax, io.err);
+    if (MODE == EPI_CORR) block_max_slot(errmax, io.err, io.err_mask);
 }
 
 // ------------------------------------------------------------------ y passes
@@ -209,8 +247,8 @@ y_comp_tile(const DemagGeom &g, const CompFFT &f, int lw, int kx0, const float2 
     load_tw(f, stw);
     const int last = g.h2 - 1 - kx0;
     stage_first<RM, DIR>(f, ln, A, [&](int w, int j, int o) {
-        const float2 *line = src + (long)j * g.sx + kx0 + min(w, last);
-        return j + o < nin ? line[(long)o * g.sx] : float2{0.0f, 0.0f};
+        const unsigned at = 8u * (unsigned)(j * g.sx + kx0 + min(w, last));
+        return j + o < nin ? ld_off<float2>(src + (long)o * g.sx, at) : float2{0.0f, 0.0f};
     });
     __syncthreads();
     if (f.ns == 3) {
@@ -218,8 +256,8 @@ y_comp_tile(const DemagGeom &g, const CompFFT &f, int lw, int kx0, const float2 
         __syncthreads();
     }
     stage_last<RM, DIR>(f, ln, A, stw, [&](int w, int q, int o, int, float2 v) {
-        float2 *line = dst + (long)q * g.sx + kx0 + w;
-        if (w <= last && q + o < nout) line[(long)o * g.sx] = v;
+        if (w <= last && q + o < nout)
+            st_off<float2>(dst + (long)o * g.sx, 8u * (unsigned)(q * g.sx + kx0 + w), v);
     });
 }
 
@@ -230,6 +268,13 @@ y_comp_tile(const DemagGeom &g, const CompFFT &f, int lw, int kx0, const float2 
 // multiply walks the slots.  (A thread that held the last stage's points of all
 // three components and multiplied them in registers saved two barriers, but at
 // 256 registers, two waves per SIMD, z of 240x200x36 took 112 us against 66.)
+
+// The three components of a line's first R1 (R2) elements lie within 4 GiB of
+// each other: 32-bit byte offsets from a scalar base.
+__host__ __device__ inline bool comp_line_fits(long cs, long es, int m0)
+{
+    return (2.0 * cs + (double)m0 * es + 4096.0) * sizeof(float2) < 4294967295.0;
+}
 
 struct CompLine {            // the transformed axis in memory
     float2 *base;            // element 0, component 0, column kx0
@@ -270,6 +315,11 @@ __device__ __forceinline__ void z_comp_tile(const DemagGeom &g, const CompFFT &f
     float2 *A = sm, *stw = sm + 3 * ln.span;
     load_tw(f, stw);
     const int last = g.h2 - 1 - c.kx0, NT = blockDim.x;
+    // byte offset of element j of line l = (component, column) from c.base
+    const unsigned cs8 = 8u * (unsigned)c.cs, es8 = 8u * (unsigned)c.es;
+    auto lane_off = [&](int l, int j, int w) {
+        return (unsigned)(l >> lw) * cs8 + (unsigned)j * es8 + 8u * (unsigned)w;
+    };
     // slot t of the W columns: its LDS element and kernel values
     auto place = [&](int t, int &o) {
         const int w = t & (W - 1), e = t >> lw;
@@ -279,8 +329,8 @@ __device__ __forceinline__ void z_comp_tile(const DemagGeom &g, const CompFFT &f
         return c.film ? kern_at(g, K, 0, k, kx) : kern_at(g, K, k, c.kfix, kx);
     };
     stage_first<RM, -1>(f, ln, A, [&](int l, int j, int o) {
-        const float2 *line = c.base + (l >> lw) * c.cs + j * c.es + min(l & (W - 1), last);
-        return j + o < c.n ? line[o * c.es] : float2{0.0f, 0.0f};
+        const unsigned at = lane_off(l, j, min(l & (W - 1), last));
+        return j + o < c.n ? ld_off<float2>(c.base + o * c.es, at) : float2{0.0f, 0.0f};
     });
     // the kernel values of a thread's first slots, their loads under the
     // remaining forward stages (four slots each cost registers: z of 240x200x36
@@ -315,8 +365,7 @@ __device__ __forceinline__ void z_comp_tile(const DemagGeom &g, const CompFFT &f
     }
     stage_first_back<RM>(f, ln, A, [&](int l, int j, int o, float2 v) {
         const int w = l & (W - 1);
-        float2 *line = c.base + (l >> lw) * c.cs + j * c.es + w;
-        if (w <= last && j + o < c.n) line[o * c.es] = v;
+        if (w <= last && j + o < c.n) st_off<float2>(c.base + o * c.es, lane_off(l, j, w), v);
     });
 }
 

@@ -1,5 +1,8 @@
 // comp_x.hip -- the x passes on composite-radix transforms (comp_tiles.hpp), one simulation, and the
 // choice of radices.
+#include <cstdint>
+#include <initializer_list>
+
 #include "comp_launch.hpp"
 
 namespace mmx {
@@ -63,25 +66,22 @@ template <int RM, int PRED>
 MMX_COMP_KERNEL xf_comp(DemagGeom g, CompFFT f, int RB, const float *__restrict__ m,
                         const float *__restrict__ msat_map, const float *__restrict__ tau0, float h,
                         const float *__restrict__ norm_map, float *__restrict__ mpred,
-                        float2 *__restrict__ xb, unsigned int *ho_dev, unsigned int *ho_host)
+                        float2 *__restrict__ xb, unsigned int *ho_dev, unsigned int *ho_host, int pairs)
 {
     extern __shared__ float2 sm[];
-    if (ho_dev != nullptr && blockIdx.x == 0 && threadIdx.x == 0) {
-        // the previous launch's result word to the host, cleared for the next
-        const unsigned int e = __hip_atomic_load(ho_dev, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(ho_host, e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-        __hip_atomic_store(ho_dev, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    xf_comp_tile<RM, PRED>(g, f, RB, (long)xcd_tile(blockIdx.x, gridDim.x) * RB, m, msat_map, tau0, h,
-                           norm_map, mpred, xb, sm);
+    // a hand-off takes a workgroup of its own, the last one
+    const int nb = gridDim.x - (ho_dev != nullptr);
+    if ((int)blockIdx.x == nb) return hand_off(ho_dev, ho_host);
+    xf_comp_tile<RM, PRED>(g, f, RB, (long)xcd_tile(blockIdx.x, nb) * RB, m, msat_map, tau0, h, norm_map,
+                           mpred, xb, sm, pairs != 0);
 }
 
-template <int RM, int MODE>
+template <int RM, int MODE, int PAIR>
 MMX_COMP_KERNEL xi_comp(DemagGeom g, CompFFT f, int RB, const float2 *__restrict__ xb, FieldParams fp,
                         EpilogueIO io)
 {
     extern __shared__ float2 sm[];
-    xi_comp_tile<RM, MODE>(g, f, RB, (long)xcd_tile(blockIdx.x, gridDim.x) * RB, xb, fp, io, sm);
+    xi_comp_tile<RM, MODE, PAIR>(g, f, RB, (long)xcd_tile(blockIdx.x, gridDim.x) * RB, xb, fp, io, sm);
 }
 
 // Rows per workgroup: as few as leave all workgroups resident at once (a row's
@@ -96,10 +96,18 @@ static int comp_rows(const DemagPlanImpl *P)
 
 bool comp_x_applies(const DemagPlanImpl *P)
 {
-    return P->cx.ns > 0 && comp_x_lds(P->cx, 1) <= kLdsMax &&
-           (P->g.n2 == P->cx.L || P->g.n2 == 2 * P->cx.L) &&
-           P->g.nrows < 2147480000L; // rows as int, the last tile's included
+    return P->cx.ns > 0 && comp_x_lds(P->cx, 1) <= kLdsMax && comp_x_fits(P->g);
 }
+
+// 8-byte accesses of cell pairs (a component starts at an even cell when n2 is
+// even; the caller's arrays may start anywhere)
+static bool aligned8(std::initializer_list<const void *> ps)
+{
+    for (const void *p : ps)
+        if (reinterpret_cast<uintptr_t>(p) % 8) return false;
+    return true;
+}
+
 template <int RM, int PRED>
 static int xf_go(const DemagPlanImpl *P, const float *m, const float *msat_map, const float *tau0, float h,
                  const float *norm_map, float *mpred, hipStream_t st)
@@ -107,9 +115,10 @@ static int xf_go(const DemagPlanImpl *P, const float *m, const float *msat_map, 
     const int rb = comp_rows(P);
     const size_t b = comp_x_lds(P->cx, rb);
     comp_lds(xf_comp<RM, PRED>, b);
-    xf_comp<RM, PRED><<<dim3(div_up(P->g.nrows, rb)), dim3(kBlock), b, st>>>(
-        P->g, P->cx, rb, m, msat_map, tau0, h, norm_map, mpred, P->xbuf, PRED ? nullptr : P->handoff_dev,
-        PRED ? nullptr : P->handoff_host);
+    unsigned int *ho = PRED ? nullptr : P->handoff_dev;
+    const bool pairs = P->g.n2 % 2 == 0 && aligned8({m, msat_map, tau0, norm_map, mpred});
+    xf_comp<RM, PRED><<<dim3(div_up(P->g.nrows, rb) + (ho ? 1 : 0)), dim3(kBlock), b, st>>>(
+        P->g, P->cx, rb, m, msat_map, tau0, h, norm_map, mpred, P->xbuf, ho, P->handoff_host, pairs);
     MMX_CHECK_LAUNCH();
     return MMX_OK;
 }
@@ -125,27 +134,47 @@ int comp_xf(const DemagPlanImpl *P, int pred, const float *m, const float *msat_
              : xf_go<32, 0>(P, m, msat_map, nullptr, 0.0f, nullptr, nullptr, st);
 }
 
-template <int RM, int MODE>
+template <int RM, int MODE, int PAIR>
 static int xi_go(const DemagPlanImpl *P, const FieldParams &fp, const EpilogueIO &io, hipStream_t st)
 {
     const int rb = comp_rows(P);
     const size_t b = comp_x_lds(P->cx, rb);
-    comp_lds(xi_comp<RM, MODE>, b);
-    xi_comp<RM, MODE><<<dim3(div_up(P->g.nrows, rb)), dim3(kBlock), b, st>>>(P->g, P->cx, rb, P->xbuf, fp,
-                                                                             io);
+    comp_lds(xi_comp<RM, MODE, PAIR>, b);
+    xi_comp<RM, MODE, PAIR><<<dim3(div_up(P->g.nrows, rb)), dim3(kBlock), b, st>>>(P->g, P->cx, rb, P->xbuf,
+                                                                                   fp, io);
     MMX_CHECK_LAUNCH();
     return MMX_OK;
+}
+
+template <int RM, int MODE>
+static int xi_pair(const DemagPlanImpl *P, int pair, const FieldParams &fp, const EpilogueIO &io,
+                   hipStream_t st)
+{
+    if constexpr (MODE == EPI_B)
+        return pair ? xi_go<RM, MODE, 1>(P, fp, io, st) : xi_go<RM, MODE, 0>(P, fp, io, st);
+    else
+        return pair == 1   ? xi_go<RM, MODE, 1>(P, fp, io, st)
+               : pair == 2 ? xi_go<RM, MODE, 2>(P, fp, io, st)
+                           : xi_go<RM, MODE, 0>(P, fp, io, st);
 }
 
 template <int RM>
 static int xi_mode(const DemagPlanImpl *P, int mode, const FieldParams &fp, const EpilogueIO &io,
                    hipStream_t st)
 {
+    // two cells at a time where the grid fills the chip: more rows than
+    // workgroups wanted (below, half as many threads would each take longer)
+    const bool even = P->g.n2 % 2 == 0 && P->g.nrows > kCompSlots &&
+                      aligned8({io.m, io.hout, io.tout, io.tau0, io.mnew});
+    const int pair = !even                                        ? 0
+                     : (mode == EPI_B || fast_xi_applies(fp))     ? 1
+                     : fast_xi_maps_applies(fp)                   ? 2
+                                                                  : 0;
     switch (mode) {
-    case EPI_B: return xi_go<RM, EPI_B>(P, fp, io, st);
-    case EPI_HEFF: return xi_go<RM, EPI_HEFF>(P, fp, io, st);
-    case EPI_TAU0: return xi_go<RM, EPI_TAU0>(P, fp, io, st);
-    case EPI_CORR: return xi_go<RM, EPI_CORR>(P, fp, io, st);
+    case EPI_B: return xi_pair<RM, EPI_B>(P, pair, fp, io, st);
+    case EPI_HEFF: return xi_pair<RM, EPI_HEFF>(P, pair, fp, io, st);
+    case EPI_TAU0: return xi_pair<RM, EPI_TAU0>(P, pair, fp, io, st);
+    case EPI_CORR: return xi_pair<RM, EPI_CORR>(P, pair, fp, io, st);
     default: set_error("demag_inverse: bad mode %d", mode); return MMX_ERR_ARG;
     }
 }

@@ -49,11 +49,15 @@ bool comp_z_applies(const DemagPlanImpl *P)
     const DemagGeom &g = P->g;
     if (g.p0 == 1) return false;
     if (zcol_applies(g) && (double)g.p1 * g.h2 + kZCols < 2147483647.0) return true;
-    return P->cz.ns > 0 && comp_z_lds(P->cz, 0) <= kLdsMax;
+    const long es = (long)g.p1 * g.sx;
+    return P->cz.ns > 0 && comp_z_lds(P->cz, 0) <= kLdsMax &&
+           comp_line_fits(g.n0 * es, es, P->cz.L / P->cz.R[0]);
 }
 bool comp_y2d_applies(const DemagPlanImpl *P)
 {
-    return P->g.p0 == 1 && P->cy.ns > 0 && comp_z_lds(P->cy, 0) <= kLdsMax;
+    const DemagGeom &g = P->g;
+    return g.p0 == 1 && P->cy.ns > 0 && comp_z_lds(P->cy, 0) <= kLdsMax &&
+           comp_line_fits(g.nrows * g.sx, g.sx, P->cy.L / P->cy.R[0]);
 }
 
 // Threads of a workgroup: the CU's waves (four per SIMD in class 16, three in

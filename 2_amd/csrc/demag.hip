@@ -35,12 +35,7 @@ xf_kernel(DemagGeom g, LineFFT<float> fx, int RB, const float *__restrict__ m,
           float2 *__restrict__ xb, unsigned int *ho_dev, unsigned int *ho_host)
 {
     extern __shared__ float2 sm[];
-    if (ho_dev != nullptr && blockIdx.x == 0 && threadIdx.x == 0) {
-        // the previous launch's result word to the host, cleared for the next
-        const unsigned int e = __hip_atomic_load(ho_dev, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(ho_host, e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-        __hip_atomic_store(ho_dev, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
+    if (ho_dev != nullptr && blockIdx.x == gridDim.x - 1) return hand_off(ho_dev, ho_host);
     xf_tile<PRED>(g, fx, RB, (long)blockIdx.x * RB, m, msat_map, tau0, h, norm_map, mpred, xb,
                   sm);
 }
@@ -96,7 +91,19 @@ xi_kernel(DemagGeom g, LineFFT<float> fx, int RB, const float2 *__restrict__ xb,
     xi_tile<MODE>(g, fx, RB, (long)blockIdx.x * RB, xb, fp, io, sm);
 }
 
+__global__ void __launch_bounds__(64) err_hand_off_kernel(unsigned int *dev, unsigned int *host)
+{
+    hand_off(dev, host);
+}
+
 // ------------------------------------------------------------ host launchers
+
+int err_hand_off(unsigned int *dev, unsigned int *host, hipStream_t st)
+{
+    err_hand_off_kernel<<<dim3(1), dim3(64), 0, st>>>(dev, host);
+    MMX_CHECK_LAUNCH();
+    return MMX_OK;
+}
 
 // Pass ids of the timed evaluation: 3-D xf 0, yf 1, z 2, yi 3, xi 4; films
 // xf 0, y2d 1, xi 2.  mark(P, st, pass) ends a launch of `pass` (-1: start).
@@ -131,6 +138,8 @@ template <typename K> static void allow_lds(K kernel, size_t bytes)
 }
 
 bool fast_length(int L) { return fast_length_impl(L); }
+bool fast_x_length(int L) { return fast_x_length_impl(L); }
+bool fast_xf_length(int L) { return fast_xf_length_impl(L); }
 bool fast_ylength(int L) { return fast_ylength_impl(L); }
 
 static int y_and_z_passes(DemagPlanImpl *P, hipStream_t st)
@@ -212,9 +221,16 @@ int set_fast_x_min_blocks(int n)
     return g_fast_x_min.exchange(n, std::memory_order_relaxed);
 }
 
-bool fast_xf_used(const DemagPlanImpl *P)
+static bool fast_x_big(const DemagPlanImpl *P) { return fast_x_blocks(P->g) >= fast_x_min_blocks(); }
+// the register-FFT x passes: grids of enough workgroups; xf of 1024 points
+// without a map, xi without the Zhang-Li torque
+static bool fast_xf_used(const DemagPlanImpl *P, const float *map)
 {
-    return P->fast_x && fast_x_blocks(P->g) >= fast_x_min_blocks();
+    return P->fast_xf && (!map || P->fast_xi) && fast_x_big(P);
+}
+static bool fast_xi_used(const DemagPlanImpl *P, int mode, const FieldParams &fp)
+{
+    return P->fast_xi && (mode == EPI_B || fast_xi_maps_applies(fp)) && fast_x_big(P);
 }
 
 int demag_forward(DemagPlanImpl *P, const float *m, const float *msat_map, hipStream_t st)
@@ -224,12 +240,12 @@ int demag_forward(DemagPlanImpl *P, const float *m, const float *msat_map, hipSt
     allow_lds(xf_kernel<0>, b);
     const int nb = div_up(g.nrows, P->tiles.rows_x);
     mark(P, st, PASS_START);
-    if (fast_xf_used(P)) {
+    if (fast_xf_used(P, msat_map)) {
         MMX_TRY(fast_xf(P, 0, m, msat_map, nullptr, 0.0f, nullptr, nullptr, st));
     } else if (comp_x_applies(P)) {
         MMX_TRY(comp_xf(P, 0, m, msat_map, nullptr, 0.0f, nullptr, nullptr, st));
     } else {
-        xf_kernel<0><<<dim3(nb), dim3(kBlock), b, st>>>(g, P->fx, P->tiles.rows_x, m, msat_map,
+        xf_kernel<0><<<dim3(nb + (P->handoff_dev ? 1 : 0)), dim3(kBlock), b, st>>>(g, P->fx, P->tiles.rows_x, m, msat_map,
                                                          nullptr, 0.0f, nullptr, nullptr, P->xbuf,
                                                          P->handoff_dev, P->handoff_host);
         MMX_CHECK_LAUNCH();
@@ -248,7 +264,7 @@ int demag_forward_pred(DemagPlanImpl *P, const float *m0, const float *tau0, flo
     const int nb = div_up(g.nrows, P->tiles.rows_x);
     // the demag source is M = m * Msat_map, norm map = Msat map
     mark(P, st, PASS_START);
-    if (fast_xf_used(P)) {
+    if (fast_xf_used(P, norm_map)) {
         MMX_TRY(fast_xf(P, 1, m0, norm_map, tau0, h, norm_map, mpred, st));
     } else if (comp_x_applies(P)) {
         MMX_TRY(comp_xf(P, 1, m0, norm_map, tau0, h, norm_map, mpred, st));
@@ -270,7 +286,7 @@ int demag_inverse(DemagPlanImpl *P, int mode, const FieldParams &fp, const Epilo
     const int nb = div_up(g.nrows, P->tiles.rows_x);
     const int RB = P->tiles.rows_x;
     const int pass_xi = (g.p0 == 1) ? 2 : 4;
-    if (P->fast_x && fast_x_blocks(g) >= fast_x_min_blocks()) {
+    if (fast_xi_used(P, mode, fp)) {
         MMX_TRY(fast_xi(P, mode, fp, io, st));
         mark(P, st, pass_xi);
         return MMX_OK;

@@ -127,7 +127,7 @@ int fast_xf(const DemagPlanImpl *P, int pred, const float *m, const float *msat_
     switch (g.Lx) {
 #define CASE(L)                                                                              \
     case L: return xf_len<L>(P, pred, m, msat_map, tau0, h, norm_map, mpred, st);
-        MMX_SHORT_LENGTHS(CASE)
+        MMX_XF_LENGTHS(CASE)
 #undef CASE
     default: set_error("fast_xf: length %d", g.Lx); return MMX_ERR_SIZE;
     }
@@ -139,7 +139,7 @@ int fast_x_blocks(const DemagGeom &g)
     switch (g.Lx) {
 #define CASE(L)                                                                              \
     case L: return div_up((int)g.nrows, RowTile<L>::R);
-        MMX_SHORT_LENGTHS(CASE)
+        MMX_XF_LENGTHS(CASE)
 #undef CASE
     default: return 0;
     }
@@ -158,16 +158,13 @@ int fast_xi(const DemagPlanImpl *P, int mode, const FieldParams &fp, const Epilo
 {
     const DemagGeom &g = P->g;
     MMX_REQUIRE(fast_x_addressable(g), MMX_ERR_SIZE, "fast_xi: unsupported geometry");
-    const int var = (mode == EPI_B || fast_xi_applies(fp)) ? XI_UNIFORM
-                    : fast_xi_maps_applies(fp)                ? XI_MAPS
-                                                              : XI_GENERAL;
+    const int var = (mode == EPI_B || fast_xi_applies(fp)) ? XI_UNIFORM : XI_MAPS;
     switch (g.Lx) {
 #define CASE(L)                                                                              \
     case L:                                                                                  \
         return var == XI_UNIFORM ? xi_len<L, XI_UNIFORM>(P, mode, fp, io, st)                \
-               : var == XI_MAPS  ? xi_len<L, XI_MAPS>(P, mode, fp, io, st)                   \
-                                 : xi_len<L, XI_GENERAL>(P, mode, fp, io, st);
-        MMX_SHORT_LENGTHS(CASE)
+                                 : xi_len<L, XI_MAPS>(P, mode, fp, io, st);
+        MMX_X_LENGTHS(CASE)
 #undef CASE
     default: set_error("fast_xi: length %d", g.Lx); return MMX_ERR_SIZE;
     }

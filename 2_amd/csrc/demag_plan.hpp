@@ -52,6 +52,12 @@ enum EpilogueMode : int {
     EPI_CORR = 3,   // RK corrector: tau1, m_new = norm(m + h/2 (tau1 - tau0)), max|tau1-tau0|
 };
 
+// The cell-independent part of the Zhang-Li torque: current direction and the
+// weights of the adiabatic and non-adiabatic terms.
+struct ZlCoef {
+    float dir[3], c_adiab, c_nonad, inv_ms;
+};
+
 // Everything the fused epilogue needs besides the demag spectrum.
 struct FieldParams {
     float demag_scale;          // Ms (H) or mu0 Ms (B)
@@ -84,6 +90,9 @@ struct FieldParams {
     const float *hdex = nullptr;
     const float *pol_map = nullptr;
     const float *xi_map = nullptr;
+    // Zhang-Li coefficients of every cell when no map varies them
+    int zl_uniform = 0;
+    ZlCoef zl_uni = {};
 };
 
 // Per-launch state of the epilogue (pointers that change between calls).
@@ -94,7 +103,8 @@ struct EpilogueIO {
     const float *tau0;    // EPI_CORR: first-stage torque
     float *mnew;          // EPI_CORR: corrected, normalised m
     float h;              // EPI_CORR: dt*gamma (float32, solve_rk12.go:153)
-    unsigned int *err;    // EPI_CORR: max |tau1 - tau0| (float bits)
+    unsigned int *err;    // EPI_CORR: max |tau1 - tau0| (float bits), in
+    unsigned int err_mask = kErrSlots - 1; // err_mask + 1 words, kErrStride apart
 };
 
 // Tunables of the pass kernels.
@@ -119,14 +129,15 @@ struct DemagPlanImpl {
     float2 *ybuf = nullptr;      // 3 x n0 x p1 x sx
     float *kern = nullptr;       // 6 x ko0 x ko1 x h2 (octant, real, 1/Np)
     float *real_kernel = nullptr;// optional: 6 x p0 p1 p2 real-space kernel
-    bool fast_x = false, fast_y = false, fast_z = false; // register-FFT passes
+    // register-FFT passes
+    bool fast_xf = false, fast_xi = false, fast_y = false, fast_z = false;
     hipEvent_t *events = nullptr; // when set: recorded before/after every launch
     int *event_pass = nullptr;    // pass id of the launch that each event ends
     int nevent = 0;
-    // Set by the caller around one demag_forward: the x pass's first thread
-    // moves the word *handoff_dev (left by the previous launch on the stream)
-    // into the pinned host word *handoff_host and clears it, and after_x is
-    // recorded once the x pass has been queued.
+    // Set by the caller around one demag_forward: a workgroup of the x pass
+    // moves the maximum of handoff_dev's kErrSlots words (left by the previous launch
+    // on the stream) into the pinned host word *handoff_host and clears them, and
+    // after_x is recorded once the x pass has been queued.
     unsigned int *handoff_dev = nullptr, *handoff_host = nullptr;
     hipEvent_t after_x = nullptr;
     // ConvPlan: the real-space kernel comes from the caller (6 host float32
@@ -163,7 +174,8 @@ int demag_inverse(DemagPlanImpl *P, int mode, const FieldParams &fp,
                   const EpilogueIO &io, hipStream_t st);
 
 // Power-of-two passes (demag_fast.hip)
-bool fast_length(int L);   // x passes, film y, z
+bool fast_length(int L);   // film y, z
+bool fast_x_length(int L), fast_xf_length(int L); // xi; xf
 bool fast_ylength(int L);  // 3-D y passes
 int fast_xf(const DemagPlanImpl *P, int pred, const float *m, const float *msat_map,
             const float *tau0, float h, const float *norm_map, float *mpred, hipStream_t st);
@@ -186,6 +198,9 @@ inline int comp_top(const CompFFT &f)
     for (int s = 0; s < f.ns; s++) t = f.R[s] > t ? f.R[s] : t;
     return t;
 }
+// Hands the error slots to the host and clears them, as the x pass of a
+// look-ahead does (handoff_dev), in a launch of its own.
+int err_hand_off(unsigned int *dev, unsigned int *host, hipStream_t st);
 // Composite-radix passes (comp_x.hip, comp_y.hip, comp_z.hip) for lengths whose
 // prime factors are at most 13; each tells whether it covers the plan's length.
 bool comp_x_applies(const DemagPlanImpl *P);
@@ -202,23 +217,20 @@ int comp_z(const DemagPlanImpl *P, hipStream_t st);
 int comp_y2d(const DemagPlanImpl *P, hipStream_t st);
 // The register-FFT x passes run when they have at least this many
 // workgroups (one per CU); below it a handful of workgroups each carry a long
-// serial chain and the generic LDS kernels, spread over more workgroups, are
-// faster (128x32x1 film: xf 8.3 against 12.5 us, xi 9.8 against 17.6 us;
-// 4x256x256, 64 workgroups: xf 13.1 against 16.3, xi 14.6 against 20.2; at
-// 16x256x256, 256 workgroups, the register passes win: xf 17.2 against 30.5).
+// serial chain and the composite-radix passes, spread over more workgroups, are
+// faster (4x256x256, 64 workgroups: xf 10.4 against 13.9, xi 12.5 against 20.2;
+// at 16x256x256, 256 workgroups, they are level: 15.8 / 19.6 against 16.6 / 23.3;
+// 64x256x256: 56 / 98 against 37 / 68).
 constexpr int kFastXMinBlocks = 256;
 // the value in force (mmx_set_fast_x_min_blocks)
 int fast_x_min_blocks();
 int set_fast_x_min_blocks(int n); // returns the previous value
-// Whether demag_forward runs the register-FFT x pass for this plan.
-bool fast_xf_used(const DemagPlanImpl *P);
 int fast_xi(const DemagPlanImpl *P, int mode, const FieldParams &fp, const EpilogueIO &io,
             hipStream_t st);
 // The fast C2R pass's two-cell epilogue covers uniform parameters
 // (fast_xi_applies) and the Msat, Aex, alpha and Ku maps, the B_ext and
 // anisU masks, the thermal field and H_dex (fast_xi_maps_applies: no
-// spin-transfer term); with the Zhang-Li torque fast_xi runs the general
-// per-cell epilogue (xi_gen.hip).
+// spin-transfer term).
 bool fast_xi_applies(const FieldParams &fp);
 bool fast_xi_maps_applies(const FieldParams &fp);
 

@@ -238,7 +238,7 @@ xi_tile(const DemagGeom &g, const LineFFT<float> &fx, int RB, long row0,
         }
         cell_epilogue<MODE>(g, fp, io, I, i, j, k, hd, errmax);
     }
-    if (MODE == EPI_CORR) block_max_to(errmax, io.err);
+    if (MODE == EPI_CORR) block_max_slot(errmax, io.err, io.err_mask);
 }
 
 } // namespace mmx

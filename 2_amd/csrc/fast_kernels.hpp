@@ -1,5 +1,5 @@
 // fast_kernels.hpp -- the demag pass kernels for power-of-two transform
-// lengths (register four-step FFTs), shared by demag_fast.hip and xi_gen.hip.
+// lengths (register four-step FFTs), shared by the files that instantiate them.
 //
 // Same five passes as demag.hip (xf, yf, z, yi, xi; films: xf, the y
 // transform with the kernel multiply on z_fast, xi) with
@@ -10,7 +10,7 @@
 // mapped to tiles XCD by XCD (xcd_tile).
 #pragma once
 
-#include "epilogue.hpp"
+#include "pair_epilogue.hpp"
 #include "reg_fft.hpp"
 
 namespace mmx {
@@ -89,17 +89,6 @@ __device__ __forceinline__ void col_inverse(float2 (&u)[Split<L>::E / Split<L>::
     for (int k1 = 0; k1 < E; k1++) v[k1] = sbuf[k1 * S + t * W + w];
     fft_reg<E, +1>(v);
     __syncthreads();
-}
-
-// *(T *)(base + off) with a 32-bit byte offset: with a wave-uniform base this
-// is one global access with a scalar base and a vector offset.
-template <typename T> __device__ __forceinline__ T ld_off(const void *base, unsigned off)
-{
-    return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(base) + off);
-}
-template <typename T> __device__ __forceinline__ void st_off(void *base, unsigned off, T v)
-{
-    *reinterpret_cast<T *>(reinterpret_cast<char *>(base) + off) = v;
 }
 
 // yf: FFT along y of the n0 nonzero planes.  FULL: periodic y (n1 == L);
@@ -558,16 +547,13 @@ xf_fast(DemagGeom g, const float2 *__restrict__ tw, const float2 *__restrict__ r
         unsigned int *ho_host)
 {
     using C = RowTile<LX>;
-    if (ho_dev != nullptr && blockIdx.x == 0 && threadIdx.x == 0) {
-        // the previous launch's result word to the host, cleared for the next
-        const unsigned int e = __hip_atomic_load(ho_dev, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(ho_host, e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-        __hip_atomic_store(ho_dev, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
+    // a hand-off takes a workgroup of its own, the last one
+    const int nb = gridDim.x - (ho_dev != nullptr);
+    if ((int)blockIdx.x == nb) return hand_off(ho_dev, ho_host);
     constexpr int NQ = FULL ? C::E : C::E / 2; // cell pairs 2 (t + T q), q < NQ
     extern __shared__ float2 sm[];
     float2 *sbuf = sm, *stw = sm + C::E * C::S, *srtw = stw + LX;
-    const int tile = xcd_tile(blockIdx.x, gridDim.x);
+    const int tile = xcd_tile(blockIdx.x, nb);
     const int r = threadIdx.x / C::T, t = threadIdx.x % C::T;
     const int row = tile * C::R + r;
     const bool ok = row < g.nrows;
@@ -648,248 +634,24 @@ xf_fast(DemagGeom g, const float2 *__restrict__ tw, const float2 *__restrict__ r
     }
 }
 
-// Two neighbouring cells (k0 even, k0 + 1 < n2) of one row at once, for
-// uniform material parameters (MAPS false) or the Msat, Aex, alpha and Ku
-// maps, the B_ext and anisU masks, the thermal field and H_dex (MAPS true),
-// and no spin-transfer term: the same per-cell arithmetic as cell_epilogue
-// (exchange6 order dim 0, dim 2, dim 1; SumUpdater order), with 8-byte loads
-// and stores of the cell pair.
-
-__device__ __forceinline__ int nb_lo(int pos, int len, int wrap)
-{
-    int lo = pos - 1;
-    lo = (lo < 0 && wrap) ? len + lo : lo;
-    return max(lo, 0);
-}
-__device__ __forceinline__ int nb_hi(int pos, int len, int wrap)
-{
-    int hi = pos + 1;
-    hi = (hi == len && wrap) ? hi - len : hi;
-    return min(hi, len - 1);
-}
-
-// Aex/Msat of the cell pair at byte offset b (div_zero(mask_unity(aex),
-// mask_unity(msat)) of exchange6_at), and of one cell
-__device__ __forceinline__ float2 lex_pair(const FieldParams &fp, unsigned b)
-{
-    const float2 a = fp.aex_map ? ld_off<float2>(fp.aex_map, b) : float2{1.0f, 1.0f};
-    const float2 s = fp.msat_map ? ld_off<float2>(fp.msat_map, b) : float2{1.0f, 1.0f};
-    return float2{div_zero(a.x, s.x), div_zero(a.y, s.y)};
-}
-__device__ __forceinline__ float lex_one(const FieldParams &fp, unsigned b)
-{
-    const float a = fp.aex_map ? ld_off<float>(fp.aex_map, b) : 1.0f;
-    const float s = fp.msat_map ? ld_off<float>(fp.msat_map, b) : 1.0f;
-    return div_zero(a, s);
-}
-
-template <int MODE, bool MAPS = false>
-__device__ __forceinline__ void pair_epilogue(const DemagGeom &g, const FieldParams &fp,
-                                              const EpilogueIO &io, unsigned I0, int i, int j,
-                                              int k0, const float hd0[3], const float hd1[3],
-                                              float &errmax)
-{
-    const size_t N = g.N;
-    const unsigned b0 = I0 * 4u; // byte offset of cell I0 in a component array
-    if (MODE == EPI_B) {
-#pragma unroll
-        for (int c = 0; c < 3; c++) st_off<float2>(io.hout + c * N, b0, float2{hd0[c], hd1[c]});
-        return;
-    }
-    const float *__restrict__ m = io.m;
-    float m0[3], m1[3], H0[3], H1[3];
-#pragma unroll
-    for (int c = 0; c < 3; c++) {
-        const float2 a = ld_off<float2>(m + c * N, b0);
-        m0[c] = a.x;
-        m1[c] = a.y;
-    }
-    // neighbour byte offsets: dim 0 (planes), dim 2 (along the row), dim 1
-    // (rows); negative steps wrap in the unsigned sum and land on valid cells
-    const int s0 = g.n1 * g.n2, s1 = g.n2;
-    const unsigned o0l = b0 + 4u * (unsigned)((nb_lo(i, g.n0, fp.pbc[0]) - i) * s0);
-    const unsigned o0h = b0 + 4u * (unsigned)((nb_hi(i, g.n0, fp.pbc[0]) - i) * s0);
-    const unsigned o1l = b0 + 4u * (unsigned)((nb_lo(j, g.n1, fp.pbc[1]) - j) * s1);
-    const unsigned o1h = b0 + 4u * (unsigned)((nb_hi(j, g.n1, fp.pbc[1]) - j) * s1);
-    const unsigned o2l = b0 + 4u * (unsigned)(nb_lo(k0, g.n2, fp.pbc[2]) - k0); // left of cell 0
-    const unsigned o2h = b0 + 4u * (unsigned)(nb_hi(k0 + 1, g.n2, fp.pbc[2]) - k0); // right of 1
-    const float p0 = fp.ex_pre * fp.ex_c[0], p1 = fp.ex_pre * fp.ex_c[1],
-                p2 = fp.ex_pre * fp.ex_c[2];
-    if constexpr (MAPS) {
-        // exchange weights: harmonic mean of the pair's and each neighbour's
-        // Aex/Msat (w<dim><lo|hi><cell>)
-        const float2 lc = lex_pair(fp, b0);
-        const float2 lzl = lex_pair(fp, o0l), lzh = lex_pair(fp, o0h);
-        const float2 lyl = lex_pair(fp, o1l), lyh = lex_pair(fp, o1h);
-        const float lxl = lex_one(fp, o2l), lxh = lex_one(fp, o2h);
-        const float w0l0 = avg_geom_zero(lc.x, lzl.x), w0h0 = avg_geom_zero(lc.x, lzh.x);
-        const float w0l1 = avg_geom_zero(lc.y, lzl.y), w0h1 = avg_geom_zero(lc.y, lzh.y);
-        const float w2l0 = avg_geom_zero(lc.x, lxl), w2h0 = avg_geom_zero(lc.x, lc.y);
-        const float w2l1 = avg_geom_zero(lc.y, lc.x), w2h1 = avg_geom_zero(lc.y, lxh);
-        const float w1l0 = avg_geom_zero(lc.x, lyl.x), w1h0 = avg_geom_zero(lc.x, lyh.x);
-        const float w1l1 = avg_geom_zero(lc.y, lyl.y), w1h1 = avg_geom_zero(lc.y, lyh.y);
-#pragma unroll
-        for (int c = 0; c < 3; c++) {
-            const float *mc = m + c * N;
-            const float2 zl = ld_off<float2>(mc, o0l), zh = ld_off<float2>(mc, o0h);
-            const float2 yl = ld_off<float2>(mc, o1l), yh = ld_off<float2>(mc, o1h);
-            const float xl = ld_off<float>(mc, o2l), xh = ld_off<float>(mc, o2h);
-            float e0 = p0 * (w0l0 * (zl.x - m0[c]) + w0h0 * (zh.x - m0[c]));
-            float e1 = p0 * (w0l1 * (zl.y - m1[c]) + w0h1 * (zh.y - m1[c]));
-            e0 += p2 * (w2l0 * (xl - m0[c]) + w2h0 * (m1[c] - m0[c]));
-            e1 += p2 * (w2l1 * (m0[c] - m1[c]) + w2h1 * (xh - m1[c]));
-            e0 += p1 * (w1l0 * (yl.x - m0[c]) + w1h0 * (yh.x - m0[c]));
-            e1 += p1 * (w1l1 * (yl.y - m1[c]) + w1h1 * (yh.y - m1[c]));
-            // B_ext mask: multiplier * map (the SumUpdater's vecMadd)
-            float hx0 = fp.hext[c], hx1 = fp.hext[c];
-            if (fp.bext_map) {
-                const float2 bm = ld_off<float2>(fp.bext_map + c * N, b0);
-                hx0 = fp.hext[c] * bm.x;
-                hx1 = fp.hext[c] * bm.y;
-            }
-            H0[c] = hd0[c] + e0 + hx0;
-            H1[c] = hd1[c] + e1 + hx1;
-        }
-    } else {
-#pragma unroll
-        for (int c = 0; c < 3; c++) {
-            const float *mc = m + c * N;
-            const float2 zl = ld_off<float2>(mc, o0l), zh = ld_off<float2>(mc, o0h);
-            const float2 yl = ld_off<float2>(mc, o1l), yh = ld_off<float2>(mc, o1h);
-            const float xl = ld_off<float>(mc, o2l), xh = ld_off<float>(mc, o2h);
-            float e0 = p0 * ((zl.x - m0[c]) + (zh.x - m0[c]));
-            float e1 = p0 * ((zl.y - m1[c]) + (zh.y - m1[c]));
-            e0 += p2 * ((xl - m0[c]) + (m1[c] - m0[c]));
-            e1 += p2 * ((m0[c] - m1[c]) + (xh - m1[c]));
-            e0 += p1 * ((yl.x - m0[c]) + (yh.x - m0[c]));
-            e1 += p1 * ((yl.y - m1[c]) + (yh.y - m1[c]));
-            H0[c] = hd0[c] + e0 + fp.hext[c];
-            H1[c] = hd1[c] + e1 + fp.hext[c];
-        }
-    }
-    // Msat of the pair (a zero Msat reads as 1 in the anisotropy constant and
-    // masks the renormalised cell)
-    float2 ms = float2{1.0f, 1.0f};
-    if constexpr (MAPS) {
-        if (fp.msat_map) ms = ld_off<float2>(fp.msat_map, b0);
-    }
-    if (fp.anis) {
-        float k = fp.ku2, k1 = fp.ku2;
-        if constexpr (MAPS) {
-            k = fp.ku2 / (ms.x == 0.0f ? 1.0f : ms.x);
-            k1 = fp.ku2 / (ms.y == 0.0f ? 1.0f : ms.y);
-            if (fp.ku_map) {
-                const float2 q = ld_off<float2>(fp.ku_map, b0);
-                k *= q.x;
-                k1 *= q.y;
-            }
-        }
-        // the anisU mask gives each cell's axis as multiplier * map
-        float u0[3] = {fp.u[0], fp.u[1], fp.u[2]}, u1[3] = {fp.u[0], fp.u[1], fp.u[2]};
-        if constexpr (MAPS) {
-            if (fp.u_map) {
-#pragma unroll
-                for (int c = 0; c < 3; c++) {
-                    const float2 um = ld_off<float2>(fp.u_map + c * N, b0);
-                    u0[c] = fp.u[c] * um.x;
-                    u1[c] = fp.u[c] * um.y;
-                }
-            }
-        }
-        const float mu0 = m0[0] * u0[0] + m0[1] * u0[1] + m0[2] * u0[2];
-        const float mu1 = m1[0] * u1[0] + m1[1] * u1[1] + m1[2] * u1[2];
-#pragma unroll
-        for (int c = 0; c < 3; c++) {
-            H0[c] += k * mu0 * u0[c];
-            H1[c] += k1 * mu1 * u1[c];
-        }
-    }
-    // H_therm, the SumUpdater's last term, then H_dex from its own
-    // convolution (demagexch with an Msat mask)
-    if constexpr (MAPS) {
-        if (fp.htherm) {
-#pragma unroll
-            for (int c = 0; c < 3; c++) {
-                const float2 t = ld_off<float2>(fp.htherm + c * N, b0);
-                H0[c] += t.x;
-                H1[c] += t.y;
-            }
-        }
-        if (fp.hdex) {
-#pragma unroll
-            for (int c = 0; c < 3; c++) {
-                const float2 t = ld_off<float2>(fp.hdex + c * N, b0);
-                H0[c] += t.x;
-                H1[c] += t.y;
-            }
-        }
-    }
-    if (io.hout) {
-#pragma unroll
-        for (int c = 0; c < 3; c++) st_off<float2>(io.hout + c * N, b0, float2{H0[c], H1[c]});
-    }
-    if (MODE == EPI_HEFF && io.tout == nullptr) return;
-    float t0[3], t1[3];
-    float2 alpha = float2{fp.alpha, fp.alpha};
-    if constexpr (MAPS) {
-        if (fp.alpha_map) {
-            const float2 a = ld_off<float2>(fp.alpha_map, b0);
-            alpha = float2{fp.alpha * a.x, fp.alpha * a.y};
-        }
-    }
-    llg_torque(m0, H0, alpha.x, t0);
-    llg_torque(m1, H1, alpha.y, t1);
-    if (io.tout) {
-#pragma unroll
-        for (int c = 0; c < 3; c++) st_off<float2>(io.tout + c * N, b0, float2{t0[c], t1[c]});
-    }
-    if (MODE == EPI_CORR) {
-        const float hh = 0.5f * io.h, mh = -0.5f * io.h;
-        float a0[3], a1[3];
-        float d = 0.0f;
-#pragma unroll
-        for (int c = 0; c < 3; c++) {
-            const float2 p = ld_off<float2>(io.tau0 + c * N, b0);
-            a0[c] = m0[c] + (hh * t0[c] + mh * p.x);
-            a1[c] = m1[c] + (hh * t1[c] + mh * p.y);
-            d = fmaxf(d, fmaxf(fabsf(t0[c] - p.x), fabsf(t1[c] - p.y)));
-        }
-        errmax = fmaxf(errmax, (d != d) ? __builtin_inff() : d);
-        const float l0 = sqrtf(a0[0] * a0[0] + a0[1] * a0[1] + a0[2] * a0[2]);
-        const float l1 = sqrtf(a1[0] * a1[0] + a1[1] * a1[1] + a1[2] * a1[2]);
-        const float s0 = (ms.x == 0.0f) ? 0.0f : 1.0f, s1 = (ms.y == 0.0f) ? 0.0f : 1.0f;
-        const float q0 = (l0 != 0.0f) ? s0 / l0 : 0.0f;
-        const float q1 = (l1 != 0.0f) ? s1 / l1 : 0.0f;
-#pragma unroll
-        for (int c = 0; c < 3; c++)
-            st_off<float2>(io.mnew + c * N, b0, float2{a0[c] * q0, a1[c] * q1});
-    }
-}
-
 // xi: C2R along x (imaginary parts of DC and Nyquist ignored), keep k < n2,
-// then the fused field / torque / RK epilogue, one of three variants:
-// XI_UNIFORM the pair epilogue for uniform parameters, XI_MAPS the pair
-// epilogue with maps and masks (Msat, Aex, alpha, Ku, B_ext, anisU), the
-// thermal field and H_dex, XI_GENERAL the per-cell epilogue (cell_epilogue:
-// all of these plus the Zhang-Li torque).  Each is
-// its own kernel: the general epilogue's register demand would otherwise set
-// the occupancy of the pair variants.
-enum XiVariant { XI_UNIFORM = 0, XI_MAPS = 1, XI_GENERAL = 2 };
+// then the fused field / torque / RK epilogue, one of two variants:
+// XI_UNIFORM the pair epilogue for uniform parameters, XI_MAPS with maps and
+// masks (Msat, Aex, alpha, Ku, B_ext, anisU), the thermal field and H_dex.  The
+// Zhang-Li torque takes the composite-radix pass (comp_x.hip), whose per-cell
+// epilogue at five waves per SIMD beats what was a third variant here at two
+// (256x256x64: 119 against 105 us).
+enum XiVariant { XI_UNIFORM = 0, XI_MAPS = 1 };
 
-// Minimum waves per SIMD the xi kernel is built for.  The map and general
-// epilogues of the power-of-two lengths up to 256 take all 256 VGPRs (one
-// wave per SIMD) when left alone; bounded to two waves they spill a few
-// dozen registers and still run faster (256-point rows at 256x256x64: Msat
-// map 146 -> 103 us, Zhang-Li 136 -> 127 us).  Longer rows, and the other
-// lengths, spill hundreds at two waves.
-template <int LX, int VAR> constexpr int xi_min_waves()
-{
-    return (VAR != XI_UNIFORM && LX <= 256 && (LX & (LX - 1)) == 0) ? 2 : 1;
-}
+// Minimum waves per SIMD the xi kernel is built for.  The map epilogue takes
+// all 256 VGPRs (one wave per SIMD) when left alone; bounded to two waves it
+// spills a few dozen registers and still runs faster (256-point rows at
+// 256x256x64 with an Msat map: 146 -> 103 us).
+template <int VAR> constexpr int xi_min_waves() { return VAR == XI_MAPS ? 2 : 1; }
 
 template <int LX, int MODE, bool FULL, int VAR>
 __global__ void __launch_bounds__(RowTile<LX>::NT)
-    __attribute__((amdgpu_waves_per_eu(xi_min_waves<LX, VAR>())))
+    __attribute__((amdgpu_waves_per_eu(xi_min_waves<VAR>())))
 xi_fast(DemagGeom g, const float2 *__restrict__ tw, const float2 *__restrict__ rtw,
         const float2 *__restrict__ xb, FieldParams fp, EpilogueIO io)
 {
@@ -952,37 +714,11 @@ xi_fast(DemagGeom g, const float2 *__restrict__ tw, const float2 *__restrict__ r
                 hd0[c] = fp.demag_scale * v[c][q].x;
                 hd1[c] = fp.demag_scale * v[c][q].y;
             }
-            if (VAR == XI_GENERAL && MODE != EPI_B) {
-                // both cells' outputs stored as float2 pairs, as the
-                // two-cell variants store them
-                const long I0 = (long)row * g.n2 + k0;
-                CellOut o0, o1;
-                cell_epilogue<MODE>(g, fp, io, I0, i, j, k0, hd0, errmax, &o0);
-                cell_epilogue<MODE>(g, fp, io, I0 + 1, i, j, k0 + 1, hd1, errmax, &o1);
-                const size_t N = g.N;
-                const unsigned b0 = (unsigned)I0 * 4u;
-                if (io.hout) {
-#pragma unroll
-                    for (int c = 0; c < 3; c++)
-                        st_off<float2>(io.hout + c * N, b0, float2{o0.h[c], o1.h[c]});
-                }
-                if (io.tout) {
-#pragma unroll
-                    for (int c = 0; c < 3; c++)
-                        st_off<float2>(io.tout + c * N, b0, float2{o0.t[c], o1.t[c]});
-                }
-                if (MODE == EPI_CORR) {
-#pragma unroll
-                    for (int c = 0; c < 3; c++)
-                        st_off<float2>(io.mnew + c * N, b0, float2{o0.mn[c], o1.mn[c]});
-                }
-            } else {
-                pair_epilogue<MODE, VAR == XI_MAPS>(g, fp, io, (unsigned)(row * g.n2 + k0), i, j,
-                                                    k0, hd0, hd1, errmax);
-            }
+            pair_epilogue<MODE, VAR == XI_MAPS>(g, fp, io, (unsigned)(row * g.n2 + k0), i, j, k0, hd0,
+                                                hd1, errmax);
         }
     }
-    if (MODE == EPI_CORR) block_max_to(errmax, io.err);
+    if (MODE == EPI_CORR) block_max_slot(errmax, io.err, io.err_mask);
 }
 
 // ------------------------------------------------------- launch helpers
@@ -1009,7 +745,10 @@ template <int L, int VAR>
 int xi_len(const DemagPlanImpl *P, int mode, const FieldParams &fp, const EpilogueIO &io,
            hipStream_t st);
 
-// the lengths of each pass (fast_pow2_length, fast_odd_short, fast_odd_long)
+// the lengths of each pass (fast_x_length_impl, fast_xf_length_impl; fast_pow2_length,
+// fast_odd_short, fast_odd_long)
+#define MMX_X_LENGTHS(X) X(8) X(16) X(32) X(64) X(128) X(256)
+#define MMX_XF_LENGTHS(X) MMX_X_LENGTHS(X) X(1024)
 #define MMX_POW2_LENGTHS(X) X(8) X(16) X(32) X(64) X(128) X(256) X(512) X(1024) X(2048)
 #define MMX_R3_SHORT(X) X(24) X(48) X(96) X(192)
 #define MMX_R5_SHORT(X) X(40) X(80)

@@ -1,7 +1,8 @@
 // fast_launch.hpp -- launchers of the register-FFT passes for one transform
 // length each.  demag_fast.hip dispatches on the plan's lengths and calls
 // them; they are instantiated by length in separate files (demag_fast.hip,
-// xi_gen.hip, fast_r3.hip, fast_r5.hip, fast_r7.hip) that compile in parallel.
+// fast_px.hip, fast_py.hip, fast_pz.hip, xi_maps.hip, fast_r3.hip, fast_r5.hip,
+// fast_r7.hip) that compile in parallel.
 #pragma once
 
 #include "fast_kernels.hpp"
@@ -24,7 +25,7 @@ int xf_len(const DemagPlanImpl *P, int pred, const float *m, const float *msat_m
     } else {
         auto kern = full ? xf_fast<L, 0, true> : xf_fast<L, 0, false>;
         allow_lds_fast(kern, C::LDS);
-        kern<<<dim3(nb), dim3(C::NT), C::LDS, st>>>(g, P->fx.tw, P->fx.rtw, m, msat_map, nullptr,
+        kern<<<dim3(nb + (P->handoff_dev ? 1 : 0)), dim3(C::NT), C::LDS, st>>>(g, P->fx.tw, P->fx.rtw, m, msat_map, nullptr,
                                                      0.0f, nullptr, nullptr, P->xbuf,
                                                      P->handoff_dev, P->handoff_host);
     }

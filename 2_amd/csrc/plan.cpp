@@ -88,7 +88,8 @@ static int plan_init(DemagPlanImpl *P, int n0, int n1, int n2, const double cell
     }
     P->cell_kernel_type = kernel_type;
     P->accuracy = accuracy;
-    P->fast_x = fast_length(g.Lx) && fast_x_addressable(g);
+    P->fast_xf = fast_xf_length(g.Lx) && fast_x_addressable(g);
+    P->fast_xi = fast_x_length(g.Lx) && fast_x_addressable(g);
     // 3-D y passes take the longer odd lengths too; films run y2d
     P->fast_y = (g.p0 == 1) ? fast_length(g.p1) : fast_ylength(g.p1);
     P->fast_z = g.p0 > 1 && fast_length(g.p0) && fast_z_addressable(g);
@@ -123,7 +124,7 @@ static int plan_init(DemagPlanImpl *P, int n0, int n1, int n2, const double cell
     // x: three small stages before two large ones on small grids, whose x passes
     // wait for each row's chain (500x125x1: 9.4 / 12.1 against 10.6 / 13.5 us;
     // 300x300x12, 3600 rows: 25.0 / 37.9 against 22.6 / 36.3)
-    P->cx = comp_plan(g.Lx, P->fx, g.nrows <= 2048 ? 16 : 32);
+    P->cx = comp_plan(g.Lx, P->fx, (g.nrows <= 2048 || g.Lx >= 512) ? 16 : 32);
     if (comp_top(P->cx) > 16) P->cx = comp_plan(g.Lx, P->fx, 32);
     P->cy = comp_plan(g.p1, P->fy, 32);
     P->cz = comp_plan(g.p0, P->fz, 32);

@@ -283,9 +283,8 @@ template <> struct Split<224> { static constexpr int T = 4, E = 56; };
 template <> struct Split<448> { static constexpr int T = 8, E = 56; };
 
 // Lengths of the register-FFT passes.  Strided y passes of 3-D grids take
-// every length above; the passes that hold three components per thread (x
-// passes, film y, and z whose LDS holds three components) only those with at
-// most 28 registers per component.
+// every length above; film y and z, whose LDS holds three components, only
+// those with at most 28 registers per component.
 inline bool fast_pow2_length(int L)
 {
     return L == 8 || L == 16 || L == 32 || L == 64 || L == 128 || L == 256 || L == 512 ||
@@ -296,6 +295,17 @@ inline bool fast_odd_short(int L)
     return L == 24 || L == 48 || L == 96 || L == 192 || L == 40 || L == 80 || L == 56 || L == 112;
 }
 inline bool fast_odd_long(int L) { return L == 384 || L == 160 || L == 320 || L == 224 || L == 448; }
+// Lengths of the register-FFT x passes.  Their threads hold all three components:
+// at 512 points and more, and at the lengths with an odd factor, one wave per
+// SIMD is left and the composite-radix passes win (xf / xi at 192x192x48: 28 /
+// 55 against 28 / 37 us, 512x512x16: 59 / 101 against 54 / 92, 2048x128x64: 619 /
+// 1477 against 301 / 452), but for xf at 1024 points without a map (1024x1024x32:
+// 405 against 441 us).
+inline bool fast_x_length_impl(int L)
+{
+    return L == 8 || L == 16 || L == 32 || L == 64 || L == 128 || L == 256;
+}
+inline bool fast_xf_length_impl(int L) { return fast_x_length_impl(L) || L == 1024; }
 inline bool fast_length_impl(int L) { return fast_pow2_length(L) || fast_odd_short(L); }
 inline bool fast_ylength_impl(int L) { return fast_length_impl(L) || fast_odd_long(L); }
 

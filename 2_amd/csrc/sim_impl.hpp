@@ -5,6 +5,11 @@
 
 #include "demag_plan.hpp"
 
+namespace mmx {
+// words of mmx_sim::derr
+constexpr int kErrImplicit = kErrSlots * kErrStride, kErrWords = kErrImplicit + 16;
+} // namespace mmx
+
 struct mmx_sim {
     int n[3] = {0, 0, 0};
     int pbc[3] = {0, 0, 0};
@@ -68,9 +73,9 @@ struct mmx_sim {
     float *tau0_spec = nullptr;
     bool spec_valid = false;
     hipEvent_t ev_err = nullptr;
-    unsigned int *derr = nullptr; // [0]: RK error; [4 .. 12]: implicit-solver maxima
-    bool derr_clear = false;      // derr[0] is known to be zero (cleared by a hand-off)
-    unsigned int *herr = nullptr; // pinned, same layout
+    unsigned int *derr = nullptr; // RK error slots; from kErrImplicit: implicit-solver maxima
+    bool derr_clear = false;      // the slots are known to be zero (cleared by a hand-off)
+    unsigned int *herr = nullptr; // pinned: [0] RK error, [4 .. 12] implicit-solver maxima
     hipStream_t st = nullptr;
 
     // learned inner-stage field (borrowed; mmx_sim_set_surrogate)

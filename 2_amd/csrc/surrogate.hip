@@ -509,7 +509,7 @@ sur_epilogue(DemagGeom g, SurGeom s, FieldParams fp, EpilogueIO io, const float 
         }
         if (MODE != EPI_B) cell_epilogue<MODE>(g, fp, io, I, i, j, k, hd, errmax);
     }
-    if (MODE == EPI_CORR) block_max_to(errmax, io.err);
+    if (MODE == EPI_CORR) block_max_slot(errmax, io.err, io.err_mask);
 }
 
 // sum (a - b)^2 and sum c^2 per block (FP64 partials)

@@ -3,7 +3,6 @@
 // Zhang-Li, the madd family and the Reductor.  Each C entry point names the
 // reference function it replaces (include/mmx.h).
 #include <mutex>
-#include <vector>
 
 #include "epilogue.hpp"
 
@@ -388,26 +387,50 @@ static int noalloc_parts(double **out)
 
 } // namespace mmx
 
+// The partials lie in pinned host memory that the workgroups store to: no copy
+// between the launch and the host's finish (a copy to pageable memory took 15 us
+// of each reduction).  Three sets, for the three components of an average.
 struct mmx_reductor {
     long n = 0;
     int blocks = 0;
-    double *dpart = nullptr;
-    std::vector<double> hpart;
+    double *hpart = nullptr; // 3 x blocks
 };
 
 namespace mmx {
 
-static int reduce_run(mmx_reductor *r, int op, const float *a, const float *b, const float *c,
-                      long n, hipStream_t st, double *out)
+// launches one reduction into partial set `set`; returns its partial count
+static int reduce_queue(mmx_reductor *r, int op, const float *a, const float *b, const float *c,
+                        long n, int set, hipStream_t st, int *count)
 {
     MMX_REQUIRE(r && a, MMX_ERR_ARG, "reductor: NULL argument");
     MMX_REQUIRE(n > 0 && n <= r->n, MMX_ERR_ARG, "reductor: size %ld outside (0, %ld]", n, r->n);
     const int nb = std::min(r->blocks, red_blocks(n));
-    launch_reduce(op, a, b, c, n, nb, st, r->dpart);
+    launch_reduce(op, a, b, c, n, nb, st, r->hpart + (size_t)set * r->blocks);
     MMX_CHECK_LAUNCH();
-    MMX_HIP(hipMemcpyAsync(r->hpart.data(), r->dpart, sizeof(double) * nb, hipMemcpyDeviceToHost, st));
+    *count = nb;
+    return MMX_OK;
+}
+
+static int reduce_run(mmx_reductor *r, int op, const float *a, const float *b, const float *c,
+                      long n, hipStream_t st, double *out)
+{
+    int nb = 0;
+    MMX_TRY(reduce_queue(r, op, a, b, c, n, 0, st, &nb));
     MMX_HIP(hipStreamSynchronize(st));
-    *out = finish_partials(op, r->hpart.data(), nb);
+    *out = finish_partials(op, r->hpart, nb);
+    return MMX_OK;
+}
+
+// sums of the three components of a vector field (component stride n), one
+// synchronisation for all
+int reductor_sum3(mmx_reductor *r, const float *v, long n, hipStream_t st, double out[3])
+{
+    int nb = 0;
+    for (int c = 0; c < 3; c++)
+        MMX_TRY(reduce_queue(r, RED_SUM, v + c * n, nullptr, nullptr, n, c, st, &nb));
+    MMX_HIP(hipStreamSynchronize(st));
+    for (int c = 0; c < 3; c++)
+        out[c] = finish_partials(RED_SUM, r->hpart + (size_t)c * r->blocks, nb);
     return MMX_OK;
 }
 
@@ -571,10 +594,10 @@ int mmx_reductor_create(mmx_reductor **r, long n)
     mmx_reductor *x = new mmx_reductor();
     x->n = n;
     x->blocks = red_blocks(n);
-    x->hpart.resize(x->blocks);
-    if (hipMalloc(&x->dpart, sizeof(double) * x->blocks) != hipSuccess) {
+    if (hipHostMalloc((void **)&x->hpart, sizeof(double) * 3 * x->blocks, hipHostMallocDefault) !=
+        hipSuccess) {
         delete x;
-        set_error("mmx_reductor_create: out of device memory");
+        set_error("mmx_reductor_create: out of pinned memory");
         return MMX_ERR_NOMEM;
     }
     *r = x;
@@ -584,7 +607,7 @@ int mmx_reductor_create(mmx_reductor **r, long n)
 int mmx_reductor_destroy(mmx_reductor *r)
 {
     if (!r) return MMX_OK;
-    (void)hipFree(r->dpart);
+    (void)hipHostFree(r->hpart);
     delete r;
     return MMX_OK;
 }

@@ -108,6 +108,8 @@ FieldParams sim_field_params(const mmx_sim *s);
 int therm_draw(unsigned long long seed, unsigned long long draw, long N, const float *alpha_map,
                const float *temp_map, const float *msat_map, float a, float b, float *out,
                hipStream_t st);
+// Sums of a vector field's components (local.hip; synchronises once).
+int reductor_sum3(mmx_reductor *r, const float *v, long n, hipStream_t st, double out[3]);
 // One fixed-point pass of the implicit solvers (implicit.hip): the next
 // iterate and, per component c, res[3c] = max|m - b|, res[3c+1] = max|b|,
 // res[3c+2] = max|m + b| (synchronises).

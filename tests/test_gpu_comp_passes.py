@@ -106,3 +106,46 @@ def test_batch_tiles(mmx, grids):
         # three steps of float32 stages of the same arithmetic in other transforms
         assert np.abs(a.getarray("m") - b.getarray("m")).max() < 5e-6
         assert a.getv("step") == b.getv("step") == 3
+
+
+# grids of more rows than workgroups wanted: the two-cell epilogue with uniform
+# parameters and with maps, and the per-cell one with the spin-transfer torque,
+# on lengths of either register class; the corrector's maximum over many
+# workgroups
+@pytest.mark.parametrize("maps", [False, True])
+@pytest.mark.parametrize("zl", [False, True])
+@pytest.mark.parametrize("n,pbc", [((11, 100, 24), (0, 0, 0)), ((2, 650, 22), (0, 0, 1)), ((3, 350, 9), (0, 1, 0))])
+def test_cells_in_pairs(mmx, n, pbc, zl, maps):
+    from oracle import oracle as O
+    print("pairs", n, pbc, zl, maps, flush=True)
+    cell = (3e-9, 4e-9, 5e-9)
+    rng = np.random.default_rng(n[1])
+    sim = mmx.Sim(n, cell, pbc)
+    kw = dict(msat=8e5, aex=1.3e-11, alpha=0.05, bext=(0.01, 0.0, 0.02), ku=4e5, anis_u=(0.6, 0.0, 0.8))
+    for k, v in (("Msat", 8e5), ("Aex", 1.3e-11), ("alpha", 0.05), ("B_ext", kw["bext"])):
+        sim.setv(k, v)
+    sim.load("anisotropy/uniaxial")
+    sim.setv("Ku", 4e5)
+    sim.setv("anisU", (0.6, 0.0, 0.8))
+    if zl:
+        sim.load("zhang-li")
+        sim.setv("j", (2e11, 0.0, 1e12))
+        sim.setv("polarisation", 0.56)
+        sim.setv("xi", 0.05)
+        kw.update(j=(2e11, 0.0, 1e12), pol=0.56, xi=0.05)
+    if maps:
+        ms = rng.uniform(0.5, 1.0, n).astype(np.float32)
+        ax = rng.uniform(0.5, 1.5, n).astype(np.float32)
+        sim.setmask("Msat", ms)
+        sim.setmask("Aex", ax)
+        kw.update(msat_map=ms, aex_map=ax)
+    m = rng.standard_normal((3,) + n).astype(np.float32)
+    sim.setarray("m", m)
+    prob = O.Problem(n, cell, pbc=pbc, **kw)
+    mo = prob.normalized(m.astype(np.float64))
+    want = prob.heff(mo)
+    # the repository's parity bar for fields, relative to the largest value
+    assert np.abs(sim.getarray("H_eff") - want).max() <= 1e-5 * np.abs(want).max()
+    e_gpu, e_orc = sim.try_step(1e-15), prob.try_step(mo, 1e-15)
+    assert abs(e_gpu - e_orc) <= 1e-4 * e_orc
+    assert np.abs(sim.getarray("m") - prob.normalized(mo)).max() <= 1e-5

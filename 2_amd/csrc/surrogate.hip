@@ -21,7 +21,7 @@
 // Training (on the GPU, by these kernels): relative squared error of the
 // residual against the exact fine field (sum d^2 / sum target^2 per sample), backward-data as the same convolution kernel with flipped
 // and transposed weights and a ReLU-mask epilogue, weight gradients as MFMA
-// products over the pixel tiles with per-tile partial sums reduced in a fixed
+// products over the pixel tiles with per-workgroup partial sums reduced in a fixed
 // order (deterministic), Adam on FP32 master weights.  The CPU oracle
 // (oracle/surrogate.py) rounds to bf16 at the same points.
 //
@@ -29,9 +29,11 @@
 // surrogate; the first stage (at the accepted m) stays exact, and every
 // `check_every` steps the exact field at the accepted m judges the surrogate's
 // there: above the tolerance the solver falls back to the exact path.
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <random>
+#include <type_traits>
 #include <vector>
 
 #include "demag_tiles.hpp"
@@ -144,230 +146,407 @@ __device__ __forceinline__ float input_channel(const SurGeom &s, const float *__
     return 0.0f;
 }
 
-// packed bf16 input [P][32] (used by training and the tests; inference packs
-// inside the first convolution)
+// Packed bf16 input [P][32] (used by training and the tests; inference packs
+// inside the first convolution).  Bound by the latency of its scattered plane
+// reads: a wave takes 64 consecutive pixels and 8 channels, so every plane is
+// read in whole lines and a pixel's 8 channels leave in one 16-byte store
+// (256x256x4: 12.6 us with one channel per thread, which read 4 pixels of 16
+// planes per wave, 8.0 us so).
 __global__ void __launch_bounds__(kBlock)
 sur_pack(SurGeom s, const float *__restrict__ m, const float *__restrict__ bc,
          bf16_t *__restrict__ x0)
 {
-    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x; // pixel * 32 + channel
     const long P = (long)s.n1 * s.n2;
-    if (t >= P * 32) return;
-    const int ch = (int)(t & 31);
-    const long p = t >> 5;
-    const int y = (int)(p / s.n2), x = (int)(p - (long)y * s.n2);
-    x0[t] = f2bf(input_channel(s, m, bc, y, x, ch));
+    const long p = (long)blockIdx.x * 64 + (threadIdx.x & 63);
+    const int q = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); // uniform plane arithmetic
+    if (p >= P) return;
+    const int y = (int)((unsigned)p / (unsigned)s.n2), x = (int)p - y * s.n2; // P < 2^31
+    unsigned w[4];
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+        w[e] = (unsigned)f2bf(input_channel(s, m, bc, y, x, 8 * q + 2 * e)) |
+               ((unsigned)f2bf(input_channel(s, m, bc, y, x, 8 * q + 2 * e + 1)) << 16);
+    *reinterpret_cast<uint4 *>(x0 + p * 32 + 8 * q) = uint4{w[0], w[1], w[2], w[3]};
 }
 
 // ------------------------------------------------------------ convolution
 
 enum { CE_RELU_BF16 = 0, CE_LINEAR_F32 = 1, CE_MASK_BF16 = 2 };
 
+__device__ __forceinline__ fl4 mfma_any(sh8 a, sh8 b, fl4 c) { return mfma_k32(a, b, c); }
+__device__ __forceinline__ fl4 mfma_any(sh4 a, sh4 b, fl4 c)
+{
+    return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, c, 0, 0, 0);
+}
+
 // out[p][co] = epilogue(sum_tap sum_ci in[p + off(tap)][ci] * wt[tap][co][ci])
-// over a 16 x 8 pixel tile per workgroup of 4 waves (2 rows each).  The MFMA
-// computes D = A B with A = weights (rows co, k = ci) and B = the input
-// (k = ci, columns = 16 pixels of a row), so each lane ends up holding 4
-// consecutive output channels of one pixel.  PACK: the input is formed from
-// (m, coarse B) instead of being read from `in`.
+// over a 16 x 8 pixel tile per workgroup of 4 waves.  The MFMA computes
+// D = A B with A = weights (rows co, k = ci) and B = the input (k = ci,
+// columns = 16 pixels of a row), so each lane ends up holding 4 consecutive
+// output channels of one pixel.  PACK: the input is formed from (m, coarse B)
+// instead of being read from `in`.
+//
+// Bound by the latency of one load - LDS - MFMA chain per workgroup (512
+// workgroups at 256x256, two per CU), not by the 36 MFMA of a wave.  A wave
+// owns 16 output channels, so its nine weight fragments are loaded from global
+// memory straight into registers while the tile is staged, and an input
+// fragment read once from LDS serves the three output rows it belongs to.
+// With the weights staged in LDS (18 KB per workgroup) and every fragment read
+// per output row: 9.0 us a layer at 256x256, so 5.6 us.
 template <int CIN, int COUT, int EPI, int PACK>
 __global__ void __launch_bounds__(kBlock)
 sur_conv(const bf16_t *__restrict__ in, const bf16_t *__restrict__ wt,
          const float *__restrict__ bias, const bf16_t *__restrict__ mask, void *__restrict__ out,
          int H, int W, SurGeom s, const float *__restrict__ m, const float *__restrict__ bc)
 {
+    static_assert(CIN == 32 || CIN == 16, "one MFMA per tap");
+    using Frag = std::conditional_t<CIN == 32, sh8, sh4>;
     constexpr int CP = CIN + 8; // LDS pitch per pixel (bf16 elements)
-    constexpr int NQ = CIN / 4;
+    constexpr int NQ = CIN / 8, TASKS = 10 * 18 * NQ, ITER = (TASKS + kBlock - 1) / kBlock;
+    constexpr int MT = COUT / 16, ROWS = 2 * MT; // output rows of a wave
     __shared__ __align__(16) bf16_t tile[10 * 18 * CP];
-    __shared__ __align__(16) bf16_t wsh[9 * COUT * CP];
     const int x0 = blockIdx.x * 16, y0 = blockIdx.y * 8;
-    for (int t = threadIdx.x; t < 10 * 18 * NQ; t += kBlock) {
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int n = lane & 15, kq = (lane >> 4) * 4, kf = (lane >> 4) * (CIN / 4);
+    const int mt = wave % MT, row0 = (wave / MT) * ROWS, co = mt * 16 + kq;
+
+    uint4 u[ITER];
+#pragma unroll
+    for (int i = 0; i < ITER; i++) {
+        const int t = threadIdx.x + i * kBlock;
         const int q = t % NQ, pc = t / NQ, cx = pc % 18, cy = pc / 18;
         const int gy = y0 + cy - 1, gx = x0 + cx - 1;
-        bf16_t v[4] = {0, 0, 0, 0};
-        if (gy >= 0 && gy < H && gx >= 0 && gx < W) {
+        u[i] = uint4{0u, 0u, 0u, 0u};
+        if (t < TASKS && gy >= 0 && gy < H && gx >= 0 && gx < W) {
             if (PACK) {
+                unsigned w[4];
 #pragma unroll
-                for (int e = 0; e < 4; e++) v[e] = f2bf(input_channel(s, m, bc, gy, gx, 4 * q + e));
+                for (int e = 0; e < 4; e++)
+                    w[e] = (unsigned)f2bf(input_channel(s, m, bc, gy, gx, 8 * q + 2 * e)) |
+                           ((unsigned)f2bf(input_channel(s, m, bc, gy, gx, 8 * q + 2 * e + 1)) << 16);
+                u[i] = uint4{w[0], w[1], w[2], w[3]};
             } else {
-                const uint2 u = *reinterpret_cast<const uint2 *>(in + ((long)gy * W + gx) * CIN + 4 * q);
-                v[0] = (bf16_t)(u.x & 0xffffu);
-                v[1] = (bf16_t)(u.x >> 16);
-                v[2] = (bf16_t)(u.y & 0xffffu);
-                v[3] = (bf16_t)(u.y >> 16);
+                u[i] = *reinterpret_cast<const uint4 *>(in + ((long)gy * W + gx) * CIN + 8 * q);
             }
         }
-        bf16_t *d = tile + (cy * 18 + cx) * CP + 4 * q;
-        *reinterpret_cast<uint2 *>(d) = uint2{(unsigned)v[0] | ((unsigned)v[1] << 16),
-                                              (unsigned)v[2] | ((unsigned)v[3] << 16)};
     }
-    for (int t = threadIdx.x; t < 9 * COUT * NQ; t += kBlock) {
-        const int q = t % NQ, r = t / NQ;
-        *reinterpret_cast<uint2 *>(wsh + r * CP + 4 * q) =
-            *reinterpret_cast<const uint2 *>(wt + (long)r * CIN + 4 * q);
+    Frag a[9];
+#pragma unroll
+    for (int tap = 0; tap < 9; tap++)
+        a[tap] = *reinterpret_cast<const Frag *>(wt + (tap * COUT + mt * 16 + n) * CIN + kf);
+#pragma unroll
+    for (int i = 0; i < ITER; i++) {
+        const int t = threadIdx.x + i * kBlock;
+        if (t < TASKS) *reinterpret_cast<uint4 *>(tile + (t / NQ) * CP + 8 * (t % NQ)) = u[i];
     }
     __syncthreads();
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int n = lane & 15, kq = (lane >> 4) * 4, kq8 = (lane >> 4) * 8;
+
+    fl4 acc[ROWS];
 #pragma unroll
-    for (int r = 0; r < 2; r++) {
-        const int row = wave * 2 + r;
-        fl4 acc[COUT / 16];
+    for (int r = 0; r < ROWS; r++) acc[r] = fl4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-        for (int mt = 0; mt < COUT / 16; mt++) acc[mt] = fl4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int ri = 0; ri < ROWS + 2; ri++) // input row row0 + ri - 1 of the tile
 #pragma unroll
-        for (int tap = 0; tap < 9; tap++) {
-            const int dy = tap / 3, dx = tap % 3;
-            const bf16_t *bp = tile + ((row + dy) * 18 + n + dx) * CP;
-            if constexpr (CIN % 32 == 0) { // 32 input channels per MFMA
+        for (int dx = 0; dx < 3; dx++) {
+            const Frag b = *reinterpret_cast<const Frag *>(tile + ((row0 + ri) * 18 + n + dx) * CP + kf);
 #pragma unroll
-                for (int kb = 0; kb < CIN; kb += 32) {
-                    const sh8 b = *reinterpret_cast<const sh8 *>(bp + kb + kq8);
-#pragma unroll
-                    for (int mt = 0; mt < COUT / 16; mt++) {
-                        const sh8 a = *reinterpret_cast<const sh8 *>(
-                            wsh + (tap * COUT + mt * 16 + n) * CP + kb + kq8);
-                        acc[mt] = mfma_k32(a, b, acc[mt]);
-                    }
-                }
-            } else { // 16 channels (the last layer's backward-data input)
-#pragma unroll
-                for (int kb = 0; kb < CIN; kb += 16) {
-                    const sh4 b = *reinterpret_cast<const sh4 *>(bp + kb + kq);
-#pragma unroll
-                    for (int mt = 0; mt < COUT / 16; mt++) {
-                        const sh4 a = *reinterpret_cast<const sh4 *>(
-                            wsh + (tap * COUT + mt * 16 + n) * CP + kb + kq);
-                        acc[mt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc[mt], 0, 0, 0);
-                    }
-                }
-            }
+            for (int dy = 0; dy < 3; dy++)
+                if (ri - dy >= 0 && ri - dy < ROWS)
+                    acc[ri - dy] = mfma_any(a[dy * 3 + dx], b, acc[ri - dy]);
         }
-        const long pix = (long)(y0 + row) * W + x0 + n;
 #pragma unroll
-        for (int mt = 0; mt < COUT / 16; mt++) {
-            const int co = mt * 16 + kq;
-            float v[4] = {acc[mt][0], acc[mt][1], acc[mt][2], acc[mt][3]};
-            if (EPI == CE_LINEAR_F32) {
+    for (int r = 0; r < ROWS; r++) {
+        const long pix = (long)(y0 + row0 + r) * W + x0 + n;
+        float v[4] = {acc[r][0], acc[r][1], acc[r][2], acc[r][3]};
+        if (EPI == CE_LINEAR_F32) {
 #pragma unroll
-                for (int e = 0; e < 4; e++) v[e] += bias[co + e];
-                *reinterpret_cast<float4 *>(reinterpret_cast<float *>(out) + pix * COUT + co) =
-                    float4{v[0], v[1], v[2], v[3]};
+            for (int e = 0; e < 4; e++) v[e] += bias[co + e];
+            *reinterpret_cast<float4 *>(reinterpret_cast<float *>(out) + pix * COUT + co) =
+                float4{v[0], v[1], v[2], v[3]};
+        } else {
+            if (EPI == CE_RELU_BF16) {
+#pragma unroll
+                for (int e = 0; e < 4; e++) v[e] = fmaxf(v[e] + bias[co + e], 0.0f);
             } else {
-                if (EPI == CE_RELU_BF16) {
+                const uint2 mk = *reinterpret_cast<const uint2 *>(mask + pix * COUT + co);
+                const bf16_t mb[4] = {(bf16_t)(mk.x & 0xffffu), (bf16_t)(mk.x >> 16),
+                                      (bf16_t)(mk.y & 0xffffu), (bf16_t)(mk.y >> 16)};
 #pragma unroll
-                    for (int e = 0; e < 4; e++) v[e] = fmaxf(v[e] + bias[co + e], 0.0f);
-                } else {
-                    const uint2 mk = *reinterpret_cast<const uint2 *>(mask + pix * COUT + co);
-                    const bf16_t mb[4] = {(bf16_t)(mk.x & 0xffffu), (bf16_t)(mk.x >> 16),
-                                          (bf16_t)(mk.y & 0xffffu), (bf16_t)(mk.y >> 16)};
-#pragma unroll
-                    for (int e = 0; e < 4; e++) v[e] = bf2f(mb[e]) > 0.0f ? v[e] : 0.0f;
-                }
-                const unsigned lo = (unsigned)f2bf(v[0]) | ((unsigned)f2bf(v[1]) << 16);
-                const unsigned hi = (unsigned)f2bf(v[2]) | ((unsigned)f2bf(v[3]) << 16);
-                *reinterpret_cast<uint2 *>(reinterpret_cast<bf16_t *>(out) + pix * COUT + co) =
-                    uint2{lo, hi};
+                for (int e = 0; e < 4; e++) v[e] = bf2f(mb[e]) > 0.0f ? v[e] : 0.0f;
             }
+            const unsigned lo = (unsigned)f2bf(v[0]) | ((unsigned)f2bf(v[1]) << 16);
+            const unsigned hi = (unsigned)f2bf(v[2]) | ((unsigned)f2bf(v[3]) << 16);
+            *reinterpret_cast<uint2 *>(reinterpret_cast<bf16_t *>(out) + pix * COUT + co) =
+                uint2{lo, hi};
         }
     }
 }
 
-// Weight and bias gradients of one layer over a 16 x 16 pixel tile:
-// part[tile][(tap*CIN + ci)*COUT + co] = sum_p dz[p][co] x[p + off(tap)][ci],
-// part[tile][9*CIN*COUT + co] = sum_p dz[p][co].  MFMA with A = dz^T (rows co,
+// The four layers' operands of the weight gradients and of the update.
+struct SurLayers {
+    const bf16_t *x[4], *dz[4]; // layer input, gradient at its linear output
+    bf16_t *wt[4], *wbt[4];     // bf16 weights, forward and backward-data order
+    int off[5];                 // first parameter of each layer (weights, then bias), and the end
+};
+constexpr int kSurSlot = 9 * 32 * 32 + 32; // partial gradients of one workgroup and layer
+// Workgroups of the weight gradients per layer: a tile each up to 128 tiles;
+// beyond, a workgroup adds up several tiles (two workgroups per CU over the
+// four layers), so the partial gradients stay below 19 MB.  256x256 with one
+// tile each and 38 MB: 18.1 us and a longer reduction, against 16.4 us.
+constexpr int kSurParts = 128;
+
+// Weight and bias gradients of one layer over 16 x 16 pixel tiles:
+// part[(tap*CIN + ci)*COUT + co] = sum_p dz[p][co] x[p + off(tap)][ci],
+// part[9*CIN*COUT + co] = sum_p dz[p][co].  MFMA with A = dz^T (rows co,
 // k = pixels) and B = the shifted input (k = pixels, columns ci).
-template <int CIN, int COUT>
-__global__ void __launch_bounds__(kBlock)
-sur_conv_wgrad(const bf16_t *__restrict__ x, const bf16_t *__restrict__ dz, float *__restrict__ part,
-               int H, int W)
+//
+// The contraction runs over pixels, so both operands are turned to
+// channel-major order on their way into LDS: a fragment (8 pixels of one
+// channel) is then one 16-byte read, where the pixel-major tile took eight
+// 2-byte reads per operand and MFMA, which was what bound the kernel.  The
+// three taps of an input row come out of one 16 + 4 byte read by register
+// shifts, and the next tile's loads fly under the products.  A wave keeps one 16 x 16 block of (co, ci) for its taps and reads
+// every dz fragment once.  Channel pitches are odd multiples of 16 bytes (no
+// bank conflicts between the 16 channels of a read).  All four layers in one
+// launch, 512 workgroups at 256x256: 77 us of four launches before, 16.4 us
+// so.  What is left is the latency of the loads (33 MB at 2 TB/s).
+constexpr int kWgRow = 24, kWgX = 18 * kWgRow + 8, kWgD = 256 + 8;
+template <int COUT>
+__device__ __forceinline__ void wgrad_tiles(const bf16_t *__restrict__ x, const bf16_t *__restrict__ dz,
+                                            float *__restrict__ dst, int H, int W, int ntile,
+                                            bf16_t *xt, bf16_t *dzt, float *bsum)
 {
-    constexpr int XP = CIN + 8, DP = COUT + 8;
-    constexpr int NQX = CIN / 4, NQD = COUT / 4;
-    __shared__ __align__(16) bf16_t xt[18 * 18 * XP];
-    __shared__ __align__(16) bf16_t dzt[256 * DP];
-    const int x0 = blockIdx.x * 16, y0 = blockIdx.y * 16;
-    const long tileid = (long)blockIdx.y * gridDim.x + blockIdx.x;
-    for (int t = threadIdx.x; t < 18 * 18 * NQX; t += kBlock) {
-        const int q = t % NQX, pc = t / NQX, cx = pc % 18, cy = pc / 18;
-        const int gy = y0 + cy - 1, gx = x0 + cx - 1;
-        uint2 u = uint2{0u, 0u};
-        if (gy >= 0 && gy < H && gx >= 0 && gx < W)
-            u = *reinterpret_cast<const uint2 *>(x + ((long)gy * W + gx) * CIN + 4 * q);
-        *reinterpret_cast<uint2 *>(xt + (cy * 18 + cx) * XP + 4 * q) = u;
-    }
-    for (int t = threadIdx.x; t < 256 * NQD; t += kBlock) {
-        const int q = t % NQD, p = t / NQD;
-        const int gy = y0 + p / 16, gx = x0 + p % 16;
-        *reinterpret_cast<uint2 *>(dzt + p * DP + 4 * q) =
-            *reinterpret_cast<const uint2 *>(dz + ((long)gy * W + gx) * COUT + 4 * q);
-    }
-    __syncthreads();
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    constexpr int CIN = 32, NQX = CIN / 4, NQD = COUT / 4;
+    constexpr int XT = 18 * 9 * NQX, XI = (XT + kBlock - 1) / kBlock; // pairs of pixels x 4 channels
+    constexpr int DT = 128 * NQD, DI = DT / kBlock;
+    // COUT 32: a wave per (mt, nt) with all three dy; 16: waves 0, 1 take dy
+    // 0 and 1, waves 2, 3 take dy 2
+    constexpr int MT = COUT / 16, NDY = MT == 2 ? 3 : 2;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int n = lane & 15, kq = (lane >> 4) * 4, kq8 = (lane >> 4) * 8;
-    constexpr int MT = COUT / 16, NT = CIN / 16, ITEMS = 9 * MT * NT;
-    float *dst = part + tileid * (long)(9 * CIN * COUT + COUT);
-    for (int it = wave; it < ITEMS; it += 4) {
-        const int tap = it / (MT * NT), mt = (it / NT) % MT, nt = it % NT;
-        const int dy = tap / 3, dx = tap % 3;
-        fl4 acc = fl4{0.0f, 0.0f, 0.0f, 0.0f};
-        // k = the tile's 256 pixels, 32 per MFMA
-#pragma unroll 4
-        for (int ks = 0; ks < 8; ks++) {
-            sh8 a, b;
+    const int nt = wave & 1, mt = MT == 2 ? wave >> 1 : 0;
+    const int dy0 = MT == 2 ? 0 : (wave >> 1) * 2;
+    fl4 acc[3 * NDY];
 #pragma unroll
-            for (int e = 0; e < 8; e++) {
-                const int p = ks * 32 + kq8 + e, py = p >> 4, px = p & 15;
-                a[e] = (short)dzt[p * DP + mt * 16 + n];
-                b[e] = (short)xt[((py + dy) * 18 + px + dx) * XP + nt * 16 + n];
+    for (int i = 0; i < 3 * NDY; i++) acc[i] = fl4{0.0f, 0.0f, 0.0f, 0.0f};
+    float sum = 0.0f;
+    const int tw = W / 16;
+    uint2 ua[XI][2], ud[DI][2];
+    auto load = [&](int tile) {
+        const int x0 = (tile % tw) * 16, y0 = (tile / tw) * 16;
+#pragma unroll
+        for (int i = 0; i < XI; i++) {
+            const int t = threadIdx.x + i * kBlock;
+            const int q = t % NQX, pp = t / NQX, cx = 2 * (pp % 9), cy = pp / 9;
+            const int gy = y0 + cy - 1;
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                const int gx = x0 + cx + h - 1;
+                ua[i][h] = uint2{0u, 0u};
+                if (t < XT && gy >= 0 && gy < H && gx >= 0 && gx < W)
+                    ua[i][h] = *reinterpret_cast<const uint2 *>(x + ((long)gy * W + gx) * CIN + 4 * q);
             }
-            acc = mfma_k32(a, b, acc);
         }
-        // D[m = co][n = ci]: lane holds co = mt*16 + kq + e, ci = nt*16 + n
 #pragma unroll
-        for (int e = 0; e < 4; e++)
-            dst[(tap * CIN + nt * 16 + n) * COUT + mt * 16 + kq + e] = acc[e];
+        for (int i = 0; i < DI; i++) {
+            const int t = threadIdx.x + i * kBlock;
+            const int q = t % NQD, p = 2 * (t / NQD);
+            const long g = (long)(y0 + p / 16) * W + x0 + p % 16;
+#pragma unroll
+            for (int h = 0; h < 2; h++)
+                ud[i][h] = *reinterpret_cast<const uint2 *>(dz + (g + h) * COUT + 4 * q);
+        }
+    };
+    load(blockIdx.x);
+    for (int tile = blockIdx.x; tile < ntile; tile += gridDim.x) {
+        if (tile != (int)blockIdx.x) __syncthreads(); // the tile before is read
+        auto put = [](bf16_t *d, int pitch, uint2 e0, uint2 e1) {
+            *reinterpret_cast<unsigned *>(d) = (e0.x & 0xffffu) | (e1.x << 16);
+            *reinterpret_cast<unsigned *>(d + pitch) = (e0.x >> 16) | (e1.x & 0xffff0000u);
+            *reinterpret_cast<unsigned *>(d + 2 * pitch) = (e0.y & 0xffffu) | (e1.y << 16);
+            *reinterpret_cast<unsigned *>(d + 3 * pitch) = (e0.y >> 16) | (e1.y & 0xffff0000u);
+        };
+#pragma unroll
+        for (int i = 0; i < XI; i++) {
+            const int t = threadIdx.x + i * kBlock;
+            const int q = t % NQX, pp = t / NQX, cx = 2 * (pp % 9), cy = pp / 9;
+            if (t < XT) put(xt + 4 * q * kWgX + cy * kWgRow + cx, kWgX, ua[i][0], ua[i][1]);
+        }
+#pragma unroll
+        for (int i = 0; i < DI; i++) {
+            const int t = threadIdx.x + i * kBlock;
+            put(dzt + 4 * (t % NQD) * kWgD + 2 * (t / NQD), kWgD, ud[i][0], ud[i][1]);
+        }
+        __syncthreads();
+        if (tile + (int)gridDim.x < ntile) load(tile + gridDim.x); // flies under the products
+        // k = the tile's 256 pixels, 32 per MFMA
+#pragma unroll 2
+        for (int ks = 0; ks < 8; ks++) {
+            const sh8 a = *reinterpret_cast<const sh8 *>(dzt + (mt * 16 + n) * kWgD + ks * 32 + kq8);
+            const bf16_t *xr = xt + (nt * 16 + n) * kWgX + (2 * ks + (kq8 >> 4) + dy0) * kWgRow + (kq8 & 15);
+#pragma unroll
+            for (int d = 0; d < NDY; d++) {
+                if (dy0 + d > 2) break; // wave-uniform
+                const uint4 w = *reinterpret_cast<const uint4 *>(xr + d * kWgRow);
+                const unsigned w4 = *reinterpret_cast<const unsigned *>(xr + d * kWgRow + 8);
+                const uint4 b1 = uint4{(w.x >> 16) | (w.y << 16), (w.y >> 16) | (w.z << 16),
+                                       (w.z >> 16) | (w.w << 16), (w.w >> 16) | (w4 << 16)};
+                const uint4 b2 = uint4{w.y, w.z, w.w, w4};
+                acc[3 * d] = mfma_k32(a, __builtin_bit_cast(sh8, w), acc[3 * d]);
+                acc[3 * d + 1] = mfma_k32(a, __builtin_bit_cast(sh8, b1), acc[3 * d + 1]);
+                acc[3 * d + 2] = mfma_k32(a, __builtin_bit_cast(sh8, b2), acc[3 * d + 2]);
+            }
+        }
+        // bias gradient: wave w sums pixels 64 w .. 64 w + 63 of channel `lane`
+        if (lane < COUT) {
+#pragma unroll
+            for (int p = 0; p < 64; p += 8) {
+                const uint4 w = *reinterpret_cast<const uint4 *>(dzt + lane * kWgD + 64 * wave + p);
+                const unsigned e[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    sum += bf2f((bf16_t)(e[i] & 0xffffu));
+                    sum += bf2f((bf16_t)(e[i] >> 16));
+                }
+            }
+        }
     }
-    // bias gradient: wave w sums pixels 64 w .. 64 w + 63 of channel `lane`,
-    // then the four partial sums in wave order
-    __shared__ float bsum[4][COUT];
-    if (lane < COUT) {
-        float sum = 0.0f;
-#pragma unroll 8
-        for (int p = 64 * wave; p < 64 * wave + 64; p++) sum += bf2f(dzt[p * DP + lane]);
-        bsum[wave][lane] = sum;
+    // D[m = co][n = ci]: lane holds co = mt*16 + kq + e, ci = nt*16 + n
+#pragma unroll
+    for (int i = 0; i < 3 * NDY; i++) {
+        const int tap = 3 * dy0 + i;
+        if (tap < 9)
+            *reinterpret_cast<float4 *>(dst + (tap * CIN + nt * 16 + n) * COUT + mt * 16 + kq) =
+                float4{acc[i][0], acc[i][1], acc[i][2], acc[i][3]};
     }
+    // the four waves' bias sums in wave order
+    if (lane < COUT) bsum[wave * 32 + lane] = sum;
     __syncthreads();
     if (threadIdx.x < COUT)
         dst[9 * CIN * COUT + threadIdx.x] =
-            ((bsum[0][threadIdx.x] + bsum[1][threadIdx.x]) + bsum[2][threadIdx.x]) +
-            bsum[3][threadIdx.x];
+            ((bsum[threadIdx.x] + bsum[32 + threadIdx.x]) + bsum[64 + threadIdx.x]) + bsum[96 + threadIdx.x];
 }
 
-// grad[e] = sum over tiles of part[tile][e] in a fixed order, with the
-// tiles split over the 16 waves of a workgroup: wave g sums tiles
+// grid: (workgroups of a layer, 4 layers)
+__global__ void __launch_bounds__(kBlock)
+sur_conv_wgrad(SurLayers ly, float *__restrict__ part, int H, int W, int ntile)
+{
+    __shared__ __align__(16) bf16_t xt[32 * kWgX];
+    __shared__ __align__(16) bf16_t dzt[32 * kWgD];
+    __shared__ float bsum[4 * 32];
+    const int l = blockIdx.y;
+    float *dst = part + ((long)l * gridDim.x + blockIdx.x) * kSurSlot;
+    if (l == 3) wgrad_tiles<16>(ly.x[3], ly.dz[3], dst, H, W, ntile, xt, dzt, bsum);
+    else wgrad_tiles<32>(ly.x[l], ly.dz[l], dst, H, W, ntile, xt, dzt, bsum);
+}
+
+struct SurAdam {
+    float lr, b1, b2, eps, c1, c2;
+};
+
+// bf16 copies of weight v at canonical place e (tap, ci, co) of layer l:
+// forward [tap][co][ci], backward-data [tap][ci][co] with the tap flipped (the
+// transposed convolution)
+__device__ __forceinline__ void put_weight(const SurLayers &ly, int l, int e, float v)
+{
+    const int lc = l == 3 ? 4 : 5, cout = 1 << lc; // 32 input channels in every layer
+    const int co = e & (cout - 1), ci = (e >> lc) & 31, tap = e >> (lc + 5);
+    const bf16_t h = f2bf(v);
+    ly.wt[l][(tap * cout + co) * 32 + ci] = h;
+    ly.wbt[l][((8 - tap) * 32 + ci) * cout + co] = h;
+}
+
+__global__ void __launch_bounds__(kBlock)
+sur_prep_weights(SurLayers ly, const float *__restrict__ params)
+{
+    const int l = blockIdx.y, e = blockIdx.x * blockDim.x + threadIdx.x;
+    if (e < 9 * 32 * (l == 3 ? 16 : 32)) put_weight(ly, l, e, params[ly.off[l] + e]);
+}
+
+// grad[e] = sum over the workgroups of part[.][e] in a fixed order, with the
+// partial gradients split over the 16 waves of a workgroup: wave g sums
 // [g per, (g + 1) per) for 64 consecutive elements, then wave 0 adds the 16
 // partial sums in wave order (deterministic; one serial chain per element
-// over all tiles was latency-bound: 98 us per layer at 256 tiles).
+// over all tiles was latency-bound: 98 us per layer at 256 tiles).  All
+// layers in one launch (grid.y), and with UPDATE the Adam step (Kingma & Ba
+// 2015) on the FP32 master parameters and the new bf16 weights follow in the
+// same thread: nine launches of 30 us at 256x256 before, one of 4.8 us so.
 constexpr int kRedGroups = 16;
+template <int UPDATE>
 __global__ void __launch_bounds__(64 * kRedGroups)
-sur_reduce_tiles(const float *__restrict__ part, int ntile, int len, float *__restrict__ grad)
+sur_reduce_update(SurLayers ly, const float *__restrict__ part, int nparts, float *__restrict__ grad,
+                  float *__restrict__ w, float *__restrict__ m1, float *__restrict__ m2, SurAdam ad)
 {
     __shared__ float ps[kRedGroups][64];
     const int lane = threadIdx.x & 63, grp = threadIdx.x >> 6;
-    const int e = blockIdx.x * 64 + lane;
-    const int per = (ntile + kRedGroups - 1) / kRedGroups;
-    const int t0 = grp * per, t1 = min(ntile, t0 + per);
+    const int l = blockIdx.y, e = blockIdx.x * 64 + lane, len = ly.off[l + 1] - ly.off[l];
+    if ((int)blockIdx.x * 64 >= len) return; // the whole workgroup
+    const int per = (nparts + kRedGroups - 1) / kRedGroups;
+    const int t0 = grp * per, t1 = min(nparts, t0 + per);
+    const float *src = part + (long)l * nparts * kSurSlot;
     float s = 0.0f;
     if (e < len) {
-#pragma unroll 4
-        for (int t = t0; t < t1; t++) s += part[(long)t * len + e];
+#pragma unroll 8
+        for (int t = t0; t < t1; t++) s += src[(long)t * kSurSlot + e];
     }
     ps[grp][lane] = s;
     __syncthreads();
     if (grp == 0 && e < len) {
         float r = 0.0f;
         for (int g = 0; g < kRedGroups; g++) r += ps[g][lane];
-        grad[e] = r;
+        const int o = ly.off[l] + e;
+        grad[o] = r;
+        if (UPDATE) {
+            const float a = ad.b1 * m1[o] + (1.0f - ad.b1) * r;
+            const float b = ad.b2 * m2[o] + (1.0f - ad.b2) * r * r;
+            m1[o] = a;
+            m2[o] = b;
+            float v = w[o];
+            v -= ad.lr * (a / ad.c1) / (sqrtf(b / ad.c2) + ad.eps);
+            w[o] = v;
+            if (e < 9 * 32 * (l == 3 ? 16 : 32)) put_weight(ly, l, e, v);
+        }
+    }
+}
+
+__device__ __forceinline__ float target_at(const SurGeom &s, const float *__restrict__ bfine,
+                                           const float *__restrict__ bc,
+                                           const float *__restrict__ tgt_direct, long p, int y, int x,
+                                           int ch)
+{
+    const int nused = 3 * s.n0;
+    if (tgt_direct) return tgt_direct[p * nused + ch];
+    const int c = ch / s.n0, i = ch - c * s.n0;
+    const long I = ((long)i * s.n1 + y) * s.n2 + x;
+    return (bfine[c * s.N + I] - bc[c * s.Nc + coarse_of(s, i, y, x)]) * s.inv_mu0ms;
+}
+
+// per-block partial sums of target^2 (16 pixels of 16 channels each).  The scale
+// of the gradients follows from their total, and a gradient rounds to bf16: one
+// unit in the total's last place already moves the weight gradients by 1e-5,
+// so the order of the sum is kept.  64 pixels of 4 channels per wave, turned
+// through LDS to the same order, took 6.5 us at 256x256x4 against 5.6 us.
+__global__ void __launch_bounds__(kBlock)
+sur_target_sq(SurGeom s, const float *__restrict__ bfine, const float *__restrict__ bc,
+              const float *__restrict__ tgt_direct, float *__restrict__ part)
+{
+    __shared__ float red[kBlock / 64];
+    const long P = (long)s.n1 * s.n2;
+    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x; // pixel * 16 + channel
+    float v2 = 0.0f;
+    if (t < P * 16 && (int)(t & 15) < 3 * s.n0) {
+        const long p = t >> 4;
+        const int y = (int)((unsigned)p / (unsigned)s.n2), x = (int)p - y * s.n2; // P < 2^31
+        const float v = target_at(s, bfine, bc, tgt_direct, p, y, x, (int)(t & 15));
+        v2 = v * v;
+    }
+    v2 = wave_sum(v2);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v2;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        float s2 = 0.0f;
+        for (int w = 0; w < kBlock / 64; w++) s2 += red[w];
+        part[blockIdx.x] = s2;
     }
 }
 
@@ -388,64 +567,37 @@ sur_reduce_one(const float *__restrict__ part, int n, float *__restrict__ out)
     if (threadIdx.x == 0) out[0] = ps[0];
 }
 
-__device__ __forceinline__ float target_at(const SurGeom &s, const float *__restrict__ bfine,
-                                           const float *__restrict__ bc,
-                                           const float *__restrict__ tgt_direct, long p, int ch)
-{
-    const int nused = 3 * s.n0;
-    if (tgt_direct) return tgt_direct[p * nused + ch];
-    const int c = ch / s.n0, i = ch - c * s.n0;
-    const int y = (int)(p / s.n2), x = (int)(p - (long)y * s.n2);
-    const long I = ((long)i * s.n1 + y) * s.n2 + x;
-    return (bfine[c * s.N + I] - bc[c * s.Nc + coarse_of(s, i, y, x)]) * s.inv_mu0ms;
-}
-
-// per-block partial sums of target^2
-__global__ void __launch_bounds__(kBlock)
-sur_target_sq(SurGeom s, const float *__restrict__ bfine, const float *__restrict__ bc,
-              const float *__restrict__ tgt_direct, float *__restrict__ part)
-{
-    __shared__ float red[kBlock / 64];
-    const long P = (long)s.n1 * s.n2;
-    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x; // pixel * 16 + channel
-    float v2 = 0.0f;
-    if (t < P * 16 && (int)(t & 15) < 3 * s.n0) {
-        const float v = target_at(s, bfine, bc, tgt_direct, t >> 4, (int)(t & 15));
-        v2 = v * v;
-    }
-    v2 = wave_sum(v2);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v2;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        float s2 = 0.0f;
-        for (int w = 0; w < kBlock / 64; w++) s2 += red[w];
-        part[blockIdx.x] = s2;
-    }
-}
-
-// d loss / d out = 2 (out - target) / sum target^2 (bf16) and per-block
-// partial sums of the squared error; *t2 = sum target^2 (device)
+// d loss / d out = 2 (out - target) / sum target^2 (bf16), *t2 = sum target^2;
+// the per-block partial sums of the squared error go to host_part (pinned
+// memory, at most kLossBlocks; a copy to pageable memory took 10 us), sum
+// target^2 behind them.  A wave takes 64 consecutive pixels and 4 of the 16
+// channels, so the target's planes are read in whole lines: 9.7 us with one
+// channel per thread, 6.6 us so at 256x256x4.
+constexpr int kLossBlocks = 1024;
 __global__ void __launch_bounds__(kBlock)
 sur_loss(SurGeom s, const float *__restrict__ out, const float *__restrict__ bfine,
          const float *__restrict__ bc, const float *__restrict__ tgt_direct,
-         const float *__restrict__ t2, bf16_t *__restrict__ gout, float *__restrict__ part)
+         const float *__restrict__ t2, bf16_t *__restrict__ gout, float *__restrict__ host_part)
 {
     __shared__ float red[kBlock / 64];
     const long P = (long)s.n1 * s.n2;
-    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x; // pixel * 16 + channel
-    const int nused = 3 * s.n0;
-    float e2 = 0.0f;
+    const int ch0 = 4 * __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nused = 3 * s.n0;
     const float gscale = 2.0f / fmaxf(*t2, 1e-30f);
-    if (t < P * 16) {
-        const int ch = (int)(t & 15);
-        const long p = t >> 4;
-        float g = 0.0f;
-        if (ch < nused) {
-            const float d = out[t] - target_at(s, bfine, bc, tgt_direct, p, ch);
-            e2 = d * d;
-            g = gscale * d;
-        }
-        gout[t] = f2bf(g);
+    float e2 = 0.0f;
+    for (long p = (long)blockIdx.x * 64 + (threadIdx.x & 63); p < P; p += (long)gridDim.x * 64) {
+        const int y = (int)((unsigned)p / (unsigned)s.n2), x = (int)p - y * s.n2;
+        const float4 o = *reinterpret_cast<const float4 *>(out + p * 16 + ch0);
+        const float ov[4] = {o.x, o.y, o.z, o.w};
+        bf16_t g[4] = {0, 0, 0, 0};
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+            if (ch0 + e < nused) {
+                const float d = ov[e] - target_at(s, bfine, bc, tgt_direct, p, y, x, ch0 + e);
+                e2 += d * d;
+                g[e] = f2bf(gscale * d);
+            }
+        *reinterpret_cast<uint2 *>(gout + p * 16 + ch0) =
+            uint2{(unsigned)g[0] | ((unsigned)g[1] << 16), (unsigned)g[2] | ((unsigned)g[3] << 16)};
     }
     e2 = wave_sum(e2);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = e2;
@@ -453,37 +605,9 @@ sur_loss(SurGeom s, const float *__restrict__ out, const float *__restrict__ bfi
     if (threadIdx.x == 0) {
         float s2 = 0.0f;
         for (int w = 0; w < kBlock / 64; w++) s2 += red[w];
-        part[blockIdx.x] = s2;
+        host_part[blockIdx.x] = s2;
+        if (blockIdx.x == 0) host_part[gridDim.x] = *t2;
     }
-}
-
-// Adam (Kingma & Ba 2015) on the FP32 master parameters
-__global__ void __launch_bounds__(kBlock)
-sur_adam(float *__restrict__ w, const float *__restrict__ g, float *__restrict__ m1,
-         float *__restrict__ m2, int n, float lr, float b1, float b2, float eps, float c1, float c2)
-{
-    const int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= n) return;
-    const float gi = g[e];
-    const float a = b1 * m1[e] + (1.0f - b1) * gi;
-    const float b = b2 * m2[e] + (1.0f - b2) * gi * gi;
-    m1[e] = a;
-    m2[e] = b;
-    w[e] -= lr * (a / c1) / (sqrtf(b / c2) + eps);
-}
-
-// bf16 copies of a layer's weights: forward [tap][co][ci], backward-data
-// [tap][ci][co] with the tap flipped (the transposed convolution)
-__global__ void __launch_bounds__(kBlock)
-sur_prep_weights(const float *__restrict__ W, int cin, int cout, bf16_t *__restrict__ wt,
-                 bf16_t *__restrict__ wbt)
-{
-    const int e = blockIdx.x * blockDim.x + threadIdx.x; // canonical (tap, ci, co)
-    if (e >= 9 * cin * cout) return;
-    const int co = e % cout, ci = (e / cout) % cin, tap = e / (cout * cin);
-    const bf16_t v = f2bf(W[e]);
-    wt[((long)tap * cout + co) * cin + ci] = v;
-    wbt[((long)(8 - tap) * cin + ci) * cout + co] = v;
 }
 
 // H_demag (A/m) = upsampled coarse B / mu0 + Ms * out, into the field epilogue;
@@ -557,6 +681,7 @@ struct mmx_surrogate {
     float *mc = nullptr, *bc = nullptr, *bfine = nullptr, *hd = nullptr;
     mmx::bf16_t *x0 = nullptr, *act[3] = {}, *gout = nullptr, *dz[3] = {};
     float *out = nullptr, *tgt = nullptr, *part = nullptr, *loss_part = nullptr;
+    float *loss_host = nullptr; // pinned: partial sums of the loss, then sum target^2
     double *norm_part = nullptr;
     float *params = nullptr, *grads = nullptr, *adam_m = nullptr, *adam_v = nullptr;
     mmx::bf16_t *wt[4] = {}, *wbt[4] = {};
@@ -583,16 +708,28 @@ void sur_free(mmx_surrogate *S)
                     S->norm_part, S->params, S->grads, S->adam_m, S->adam_v, S->wt[0], S->wt[1],
                     S->wt[2], S->wt[3], S->wbt[0], S->wbt[1], S->wbt[2], S->wbt[3]};
     for (void *p : ptrs) (void)hipFree(p);
+    if (S->loss_host) (void)hipHostFree(S->loss_host);
     if (S->cplan) plan_destroy(S->cplan);
+}
+
+SurLayers sur_layers(const mmx_surrogate *S)
+{
+    SurLayers ly{};
+    for (int l = 0; l < 4; l++) {
+        ly.x[l] = l == 0 ? S->x0 : S->act[l - 1];
+        ly.dz[l] = l == 3 ? S->gout : S->dz[l];
+        ly.wt[l] = S->wt[l];
+        ly.wbt[l] = S->wbt[l];
+        ly.off[l] = S->off_w[l];
+    }
+    ly.off[4] = S->np;
+    return ly;
 }
 
 int prep_weights(mmx_surrogate *S, hipStream_t st)
 {
-    for (int l = 0; l < 4; l++) {
-        const int n = 9 * kSurCh[l] * kSurCh[l + 1];
-        sur_prep_weights<<<dim3(div_up(n, kBlock)), dim3(kBlock), 0, st>>>(
-            S->params + S->off_w[l], kSurCh[l], kSurCh[l + 1], S->wt[l], S->wbt[l]);
-    }
+    sur_prep_weights<<<dim3(div_up(9 * 32 * 32, kBlock), 4), dim3(kBlock), 0, st>>>(sur_layers(S),
+                                                                                    S->params);
     MMX_CHECK_LAUNCH();
     return MMX_OK;
 }
@@ -619,62 +756,53 @@ int net_forward(mmx_surrogate *S, bool pack, const float *m, hipStream_t st)
     return MMX_OK;
 }
 
+// workgroups of the loss, partial gradients of a layer
+int loss_blocks(long P) { return (int)std::min<long>(div_up(P, 64), kLossBlocks); }
+int grad_parts(int H, int W) { return std::min((H / 16) * (W / 16), kSurParts); }
+
 // loss (given the target: exact fine B + coarse B, or a direct target),
-// backward, gradients into S->grads; *loss = mean squared error
-int net_backward(mmx_surrogate *S, const float *tgt_direct, double *loss, hipStream_t st)
+// backward, gradients into S->grads and, for lr > 0, the Adam step;
+// *loss = mean squared error
+int net_backward(mmx_surrogate *S, const float *tgt_direct, float lr, double *loss, hipStream_t st)
 {
-    const long n16 = S->P * 16;
-    const int nlb = (int)div_up(n16, kBlock);
-    float *t2 = S->loss_part + nlb; // sum target^2 (one float after the partials)
-    sur_target_sq<<<dim3(nlb), dim3(kBlock), 0, st>>>(S->s, S->bfine, S->bc, tgt_direct, S->loss_part);
-    sur_reduce_one<<<dim3(1), dim3(1024), 0, st>>>(S->loss_part, nlb, t2);
+    const int nlb = loss_blocks(S->P);
+    const int ntp = (int)(S->P / 16); // partial sums of target^2, their total behind them
+    float *t2 = S->loss_part + ntp;
+    sur_target_sq<<<dim3(ntp), dim3(kBlock), 0, st>>>(S->s, S->bfine, S->bc, tgt_direct, S->loss_part);
+    sur_reduce_one<<<dim3(1), dim3(1024), 0, st>>>(S->loss_part, ntp, t2);
     sur_loss<<<dim3(nlb), dim3(kBlock), 0, st>>>(S->s, S->out, S->bfine, S->bc, tgt_direct, t2,
-                                                 S->gout, S->loss_part);
+                                                 S->gout, S->loss_host);
     const dim3 grid(S->W / 16, S->H / 8), blk(kBlock);
-    const dim3 wgrid(S->W / 16, S->H / 16);
-    const int ntile = (S->W / 16) * (S->H / 16);
-    const bf16_t *xin[4] = {S->x0, S->act[0], S->act[1], S->act[2]};
-    // layer 3 (32 -> 16): weight gradient, then d act[2]
-    sur_conv_wgrad<32, 16><<<wgrid, blk, 0, st>>>(xin[3], S->gout, S->part, S->H, S->W);
-    int len = 9 * 32 * 16 + 16;
-    sur_reduce_tiles<<<dim3(div_up(len, 64)), dim3(64 * kRedGroups), 0, st>>>(
-        S->part, ntile, len, S->grads + S->off_w[3]);
     sur_conv<16, 32, CE_MASK_BF16, 0><<<grid, blk, 0, st>>>(S->gout, S->wbt[3], nullptr, S->act[2],
                                                             S->dz[2], S->H, S->W, S->s, nullptr, nullptr);
-    for (int l = 2; l >= 0; l--) {
-        sur_conv_wgrad<32, 32><<<wgrid, blk, 0, st>>>(xin[l], S->dz[l], S->part, S->H, S->W);
-        len = 9 * 32 * 32 + 32;
-        sur_reduce_tiles<<<dim3(div_up(len, 64)), dim3(64 * kRedGroups), 0, st>>>(
-            S->part, ntile, len, S->grads + S->off_w[l]);
-        if (l > 0)
-            sur_conv<32, 32, CE_MASK_BF16, 0><<<grid, blk, 0, st>>>(
-                S->dz[l], S->wbt[l], nullptr, S->act[l - 1], S->dz[l - 1], S->H, S->W, S->s, nullptr,
-                nullptr);
+    for (int l = 2; l > 0; l--)
+        sur_conv<32, 32, CE_MASK_BF16, 0><<<grid, blk, 0, st>>>(
+            S->dz[l], S->wbt[l], nullptr, S->act[l - 1], S->dz[l - 1], S->H, S->W, S->s, nullptr, nullptr);
+    // weight gradients of all layers from the kept inputs and output gradients
+    const SurLayers ly = sur_layers(S);
+    const int ntile = (S->W / 16) * (S->H / 16), nparts = grad_parts(S->H, S->W);
+    sur_conv_wgrad<<<dim3(nparts, 4), blk, 0, st>>>(ly, S->part, S->H, S->W, ntile);
+    const dim3 rgrid(div_up(kSurSlot, 64), 4), rblk(64 * kRedGroups);
+    if (lr > 0) {
+        S->adam_t++;
+        SurAdam ad{lr, 0.9f, 0.999f, 1e-8f, 0.0f, 0.0f};
+        ad.c1 = 1.0f - (float)std::pow(0.9, (double)S->adam_t);
+        ad.c2 = 1.0f - (float)std::pow(0.999, (double)S->adam_t);
+        sur_reduce_update<1><<<rgrid, rblk, 0, st>>>(ly, S->part, nparts, S->grads, S->params, S->adam_m,
+                                                     S->adam_v, ad);
+    } else {
+        sur_reduce_update<0><<<rgrid, rblk, 0, st>>>(ly, S->part, nparts, S->grads, S->params, S->adam_m,
+                                                     S->adam_v, SurAdam{});
     }
     MMX_CHECK_LAUNCH();
     if (loss) {
-        std::vector<float> lp(nlb + 1);
-        MMX_HIP(hipMemcpyAsync(lp.data(), S->loss_part, sizeof(float) * (nlb + 1),
-                               hipMemcpyDeviceToHost, st));
         MMX_HIP(hipStreamSynchronize(st));
         double sum = 0.0;
-        for (int b = 0; b < nlb; b++) sum += lp[b];
-        *loss = lp[nlb] > 0 ? sum / (double)lp[nlb] : 0.0;
+        for (int b = 0; b < nlb; b++) sum += S->loss_host[b];
+        const double t2 = S->loss_host[nlb];
+        *loss = t2 > 0 ? sum / t2 : 0.0;
     }
     return MMX_OK;
-}
-
-int adam_step(mmx_surrogate *S, float lr, hipStream_t st)
-{
-    S->adam_t++;
-    const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
-    const float c1 = 1.0f - (float)std::pow(0.9, (double)S->adam_t);
-    const float c2 = 1.0f - (float)std::pow(0.999, (double)S->adam_t);
-    sur_adam<<<dim3(div_up(S->np, kBlock)), dim3(kBlock), 0, st>>>(S->params, S->grads, S->adam_m,
-                                                                    S->adam_v, S->np, lr, b1, b2,
-                                                                    eps, c1, c2);
-    MMX_CHECK_LAUNCH();
-    return prep_weights(S, st);
 }
 
 // coarse m (optionally from the RK predictor) and coarse B
@@ -777,7 +905,6 @@ int mmx_surrogate_create(mmx_surrogate **sur, mmx_sim *sim, unsigned long long s
     const int zero[3] = {0, 0, 0};
     int rc = plan_create(&S->cplan, s.c0, s.c1, s.c2, ccell, zero, sim->kernel_type, sim->accuracy);
     const long P = S->P;
-    const int ntile = (n2 / 16) * (n1 / 16);
     if (rc == MMX_OK) rc = dalloc(&S->mc, 3 * s.Nc);
     if (rc == MMX_OK) rc = dalloc(&S->bc, 3 * s.Nc);
     if (rc == MMX_OK) rc = dalloc(&S->bfine, 3 * s.N);
@@ -788,8 +915,12 @@ int mmx_surrogate_create(mmx_surrogate **sur, mmx_sim *sim, unsigned long long s
     if (rc == MMX_OK) rc = dalloc(&S->gout, P * 16);
     if (rc == MMX_OK) rc = dalloc(&S->out, P * 16);
     if (rc == MMX_OK) rc = dalloc(&S->tgt, P * 3 * n0);
-    if (rc == MMX_OK) rc = dalloc(&S->part, (size_t)ntile * (9 * 32 * 32 + 32));
-    if (rc == MMX_OK) rc = dalloc(&S->loss_part, (size_t)div_up(P * 16, kBlock) + 1);
+    if (rc == MMX_OK) rc = dalloc(&S->part, (size_t)4 * grad_parts(n1, n2) * kSurSlot);
+    if (rc == MMX_OK) rc = dalloc(&S->loss_part, P / 16 + 1);
+    if (rc == MMX_OK && hipHostMalloc(&S->loss_host, sizeof(float) * (loss_blocks(P) + 1)) != hipSuccess) {
+        set_error("surrogate: cannot allocate pinned memory");
+        rc = MMX_ERR_NOMEM;
+    }
     if (rc == MMX_OK) rc = dalloc(&S->norm_part, 2 * 512);
     if (rc == MMX_OK) rc = dalloc(&S->params, S->np);
     if (rc == MMX_OK) rc = dalloc(&S->grads, S->np);
@@ -891,7 +1022,7 @@ int mmx_surrogate_net(mmx_surrogate *sur, const float *x_host, const float *tgt_
     MMX_TRY(net_forward(S, false, nullptr, st));
     if (tgt_host) {
         MMX_HIP(hipMemcpyAsync(S->tgt, tgt_host, sizeof(float) * P * 3 * S->s.n0, hipMemcpyHostToDevice, st));
-        MMX_TRY(net_backward(S, S->tgt, loss, st));
+        MMX_TRY(net_backward(S, S->tgt, 0.0f, loss, st));
     }
     MMX_HIP(hipMemcpyAsync(out_host, S->out, sizeof(float) * P * 16, hipMemcpyDeviceToHost, st));
     MMX_HIP(hipStreamSynchronize(st));
@@ -910,13 +1041,10 @@ int mmx_surrogate_train_step(mmx_surrogate *sur, const float *m_dev, float lr, d
     MMX_TRY(mmx_demag_update_b(x->plan, S->bfine, S->bfine + N, S->bfine + 2 * N, m_dev, m_dev + N,
                                m_dev + 2 * N, nullptr, (float)x->msat, st));
     MMX_TRY(coarse_field(S, m_dev, nullptr, 0.0f, nullptr, st));
-    const int np32 = (int)div_up(S->P * 32, kBlock);
-    sur_pack<<<dim3(np32), dim3(kBlock), 0, st>>>(S->s, m_dev, S->bc, S->x0);
+    sur_pack<<<dim3((unsigned)div_up(S->P, 64)), dim3(kBlock), 0, st>>>(S->s, m_dev, S->bc, S->x0);
     MMX_CHECK_LAUNCH();
     MMX_TRY(net_forward(S, false, nullptr, st));
-    MMX_TRY(net_backward(S, nullptr, loss, st));
-    if (lr > 0) MMX_TRY(adam_step(S, lr, st));
-    return MMX_OK;
+    return net_backward(S, nullptr, lr, loss, st);
 }
 
 int mmx_surrogate_predict_b(mmx_surrogate *sur, const float *m_dev, float *b_dev, int coarse_only)

@@ -177,17 +177,31 @@ yi_fast(DemagGeom g, int ntx, const float2 *__restrict__ tw, const float2 *__res
 // (a DPP swap) and lanes of one row still cover W neighbouring columns.
 // Twiddles W_L^j = A[j / E] B[j % E] from two tables of T and E entries.
 
-template <int L> struct PairTile {
+// Two tiles.  4 columns with a complex exchange buffer: 69 KB, two workgroups
+// of four waves per CU; the 32 lanes of a b64 access hit distinct bank pairs in
+// both directions (T W + 2 W = 2 W mod 32).  SPLIT, 8 columns (64-byte row
+// segments): real and imaginary parts cross one after the other through a
+// buffer of floats, which leaves room for four waves per SIMD (128 registers)
+// at the price of three more barriers; the 64 lanes of a b32 access hit distinct
+// banks (T W + 2 W = 2 W mod 64).
+//
+// yi takes the split tile when that gives every CU a workgroup
+// (kPairSplitBlocks): 716 -> 602 us at 1024x1024x32, 31 -> 29 us at 64x1024x16
+// (432 workgroups), but 18.6 -> 19.3 us at 100x1024x4 (156).  yf keeps the
+// complex one: split it spills 40 registers at 128 (765 -> 987 us at
+// 1024x1024x32), and with 4 split columns at three waves it has more 32-byte
+// segments in flight than the L2 merges (851 us).
+template <int L, bool SPLIT> struct PairTile {
     static constexpr int T = 64;
     static constexpr int E = L / T;
-    static constexpr int W = 4;                // columns per workgroup
-    static constexpr int NT = T * W;           // 256 threads
-    // row pitch of the exchange: the 32 lanes of a b64 access hit distinct
-    // bank pairs in both directions (T W + 2 W = 2 W mod 32)
-    static constexpr int S = T * W + 2 * W;
-    static constexpr int LDS = (E * S + T + E) * 8;
+    static constexpr int W = SPLIT ? 8 : 4;    // columns per workgroup
+    static constexpr int NT = T * W;
+    static constexpr int WAVES = SPLIT ? 4 : 2; // per SIMD
+    static constexpr int S = T * W + 2 * W;    // row pitch of the exchange
+    static constexpr int LDS = (T + E) * 8 + E * S * (SPLIT ? 4 : 8);
     static_assert(L == 2048 && E == T / 2, "pair split: E = T / 2");
 };
+constexpr int kPairSplitBlocks = 256;
 
 // swap values between lanes 2i and 2i+1 (DPP quad_perm [1, 0, 3, 2])
 __device__ __forceinline__ float2 pair_swap(float2 v)
@@ -202,25 +216,25 @@ __device__ __forceinline__ float2 pair_swap(float2 v)
 template <int L>
 __device__ __forceinline__ float2 pair_tw(const float2 *sa, const float2 *sb, int j)
 {
-    constexpr int E = PairTile<L>::E;
+    constexpr int E = PairTile<L, false>::E;
     return cmul(sa[j / E], sb[j % E]);
 }
 
 template <int L>
 __device__ __forceinline__ void pair_tables(const float2 *__restrict__ tw, float2 *sa, float2 *sb)
 {
-    using C = PairTile<L>;
-    for (int q = threadIdx.x; q < C::T; q += C::NT) sa[q] = tw[C::E * q];
-    for (int q = threadIdx.x; q < C::E; q += C::NT) sb[q] = tw[q];
+    using C = PairTile<L, false>;
+    for (int q = threadIdx.x; q < C::T; q += blockDim.x) sa[q] = tw[C::E * q];
+    for (int q = threadIdx.x; q < C::E; q += blockDim.x) sb[q] = tw[q];
 }
 
 // yf of length 2048 on the pair split; FULL and the zero-padded rows as yf_fast
 template <int L, bool FULL>
-__global__ void __launch_bounds__(PairTile<L>::NT)
+__global__ void __launch_bounds__((PairTile<L, false>::NT))
 yf_pair(DemagGeom g, int ntx, const float2 *__restrict__ tw, const float2 *__restrict__ xb,
         float2 *__restrict__ yb)
 {
-    using C = PairTile<L>;
+    using C = PairTile<L, false>;
     constexpr int T = C::T, E = C::E, NQ = FULL ? E : E / 2;
     extern __shared__ float2 sm[];
     float2 *sbuf = sm, *sa = sm + E * C::S, *sb = sa + T;
@@ -265,15 +279,15 @@ yf_pair(DemagGeom g, int ntx, const float2 *__restrict__ tw, const float2 *__res
 }
 
 // yi of length 2048 on the pair split: the steps of yf_pair reversed
-template <int L, bool FULL>
-__global__ void __launch_bounds__(PairTile<L>::NT)
+template <int L, bool FULL, bool SPLIT>
+__global__ void __launch_bounds__((PairTile<L, SPLIT>::NT), (PairTile<L, SPLIT>::WAVES))
 yi_pair(DemagGeom g, int ntx, const float2 *__restrict__ tw, const float2 *__restrict__ yb,
         float2 *__restrict__ xb)
 {
-    using C = PairTile<L>;
+    using C = PairTile<L, SPLIT>;
     constexpr int T = C::T, E = C::E, NQ = FULL ? E : E / 2;
     extern __shared__ float2 sm[];
-    float2 *sbuf = sm, *sa = sm + E * C::S, *sb = sa + T;
+    float2 *sa = sm, *sb = sa + T, *sbuf = sb + E;
     const int tile = xcd_tile(blockIdx.x, gridDim.x);
     const int tx = tile % ntx, rest = tile / ntx, i = rest % g.n0, c = rest / g.n0;
     const int s = threadIdx.x & 1, w = (threadIdx.x >> 1) % C::W, p = (threadIdx.x >> 1) / C::W;
@@ -299,13 +313,30 @@ yi_pair(DemagGeom g, int ntx, const float2 *__restrict__ tw, const float2 *__res
 #pragma unroll
     for (int m = 0; m < E; m++) {
         const int tt = 2 * m + s;
-        const float2 x = (m == 0 && s == 0) ? u[m] : cmulc(u[m], pair_tw<L>(sa, sb, tt * p));
-        sbuf[p * C::S + tt * C::W + w] = x;
+        if (m != 0 || s != 0) u[m] = cmulc(u[m], pair_tw<L>(sa, sb, tt * p));
     }
-    __syncthreads();
+    const int put = p * C::S + s * C::W + w, get = t * C::W + w;
     float2 v[E];
+    if constexpr (SPLIT) {
+        float *fb = reinterpret_cast<float *>(sbuf);
 #pragma unroll
-    for (int k1 = 0; k1 < E; k1++) v[k1] = sbuf[k1 * C::S + t * C::W + w];
+        for (int m = 0; m < E; m++) fb[put + 2 * m * C::W] = u[m].x;
+        __syncthreads();
+#pragma unroll
+        for (int k1 = 0; k1 < E; k1++) v[k1].x = fb[get + k1 * C::S];
+        __syncthreads();
+#pragma unroll
+        for (int m = 0; m < E; m++) fb[put + 2 * m * C::W] = u[m].y;
+        __syncthreads();
+#pragma unroll
+        for (int k1 = 0; k1 < E; k1++) v[k1].y = fb[get + k1 * C::S];
+    } else {
+#pragma unroll
+        for (int m = 0; m < E; m++) sbuf[put + 2 * m * C::W] = u[m];
+        __syncthreads();
+#pragma unroll
+        for (int k1 = 0; k1 < E; k1++) v[k1] = sbuf[get + k1 * C::S];
+    }
     fft_reg<E, +1>(v);
     if (!ok) return;
     float2 *dst = xb + ((size_t)c * g.nrows + (size_t)i * g.n1) * g.sx;

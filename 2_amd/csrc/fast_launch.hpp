@@ -37,7 +37,7 @@ template <int L> int yf_len(const DemagPlanImpl *P, hipStream_t st)
 {
     const DemagGeom &g = P->g;
     if constexpr (L == 2048) {
-        using C = PairTile<L>;
+        using C = PairTile<L, false>;
         const int ntx = div_up(g.h2, C::W);
         auto kern = (g.n1 == g.p1) ? yf_pair<L, true> : yf_pair<L, false>;
         allow_lds_fast(kern, C::LDS);
@@ -59,12 +59,19 @@ template <int L> int yi_len(const DemagPlanImpl *P, hipStream_t st)
 {
     const DemagGeom &g = P->g;
     if constexpr (L == 2048) {
-        using C = PairTile<L>;
-        const int ntx = div_up(g.h2, C::W);
-        auto kern = (g.n1 == g.p1) ? yi_pair<L, true> : yi_pair<L, false>;
-        allow_lds_fast(kern, C::LDS);
-        kern<<<dim3(ntx * g.n0 * 3), dim3(C::NT), C::LDS, st>>>(g, ntx, P->fy.tw, P->ybuf,
-                                                                 P->xbuf);
+        auto launch = [&](auto split) {
+            constexpr bool SPLIT = decltype(split)::value;
+            using C = PairTile<L, SPLIT>;
+            const int ntx = div_up(g.h2, C::W);
+            auto kern = (g.n1 == g.p1) ? yi_pair<L, true, SPLIT> : yi_pair<L, false, SPLIT>;
+            allow_lds_fast(kern, C::LDS);
+            kern<<<dim3(ntx * g.n0 * 3), dim3(C::NT), C::LDS, st>>>(g, ntx, P->fy.tw, P->ybuf,
+                                                                     P->xbuf);
+        };
+        if ((long)div_up(g.h2, PairTile<L, true>::W) * g.n0 * 3 >= kPairSplitBlocks)
+            launch(std::true_type{});
+        else
+            launch(std::false_type{});
         MMX_CHECK_LAUNCH();
         return MMX_OK;
     }

@@ -2,7 +2,7 @@
 // transform lengths.  The kernels are in fast_kernels.hpp, the launchers of
 // one length in fast_launch.hpp, instantiated by length in files that compile
 // in parallel: fast_px.hip (x passes), fast_py.hip (y), fast_pz.hip (z) and
-// xi_gen.hip (the general xi epilogue) for the powers of two, fast_r3.hip,
+// xi_maps.hip (xi with parameter maps) for the powers of two, fast_r3.hip,
 // fast_r5.hip and fast_r7.hip for the lengths with a factor 3, 5 or 7.  This
 // file sees only the launchers' declarations, so it instantiates none.
 #include "fast_kernels.hpp"

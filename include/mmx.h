@@ -206,7 +206,7 @@ int mmx_demag_update_b(mmx_demag_plan *plan, float *bx, float *by, float *bz,
 
 /* Tuning of the demag x passes (no counterpart in the reference, whose FFT is
  * cuFFT's choice): the register-FFT x passes run when they span at least
- * `nblocks` workgroups, smaller grids take the generic LDS passes (faster
+ * `nblocks` workgroups, smaller grids take the composite-radix passes (faster
  * there: fewer, longer serial chains otherwise).  Default 256; 0 runs the
  * register passes wherever their lengths allow.  Process-wide; *previous (if
  * not NULL) receives the value it replaces. */

@@ -447,6 +447,18 @@ __global__ void __launch_bounds__(kBlock) newell_expand(const double *__restrict
     }
 }
 
+// The statistics of a build, one word each in a cache line of its own:
+// workgroups merging into one line run one after another, about 10 ns each.
+// That was all the time of the maximum kernels (75 us of maxabs_kernel, 26 us
+// of each extract_octant at any size up to 200x200x5, with 1024 workgroups per
+// component and every word in one line; 15 and 8 us so), hence also no more
+// workgroups than 4 values per thread need (stat_blocks).
+constexpr int kStats = 11, kStatStride = 16;
+static int stat_blocks(long n, int most)
+{
+    return (int)std::max(1L, std::min((long)most, (n + 4 * kBlock - 1) / (4 * kBlock)));
+}
+
 // max |oct[6 t + c]| per component c into dst[c] (float bits)
 __global__ void __launch_bounds__(kBlock) maxabs_oct6(const double *__restrict__ oct, long ne,
                                                       unsigned int *dst)
@@ -455,7 +467,7 @@ __global__ void __launch_bounds__(kBlock) maxabs_oct6(const double *__restrict__
     for (long t = (long)blockIdx.x * blockDim.x + threadIdx.x; t < ne; t += (long)gridDim.x * blockDim.x)
         for (int c = 0; c < 6; c++) m[c] = fmaxf(m[c], (float)fabs(oct[6 * t + c]));
     for (int c = 0; c < 6; c++) {
-        block_max_to(m[c], dst + c);
+        block_max_to(m[c], dst + c * kStatStride);
         __syncthreads();
     }
 }
@@ -491,7 +503,7 @@ __global__ void __launch_bounds__(kBlock) maxabs_kernel(const float *__restrict_
                                                         unsigned int *dst)
 {
     a += blockIdx.y * n;
-    dst += blockIdx.y;
+    dst += blockIdx.y * kStatStride;
     float m = 0.0f;
     for (long t = (long)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += (long)gridDim.x * blockDim.x)
         m = fmaxf(m, fabsf(a[t]));
@@ -584,9 +596,17 @@ __global__ void __launch_bounds__(kBlock) extract_octant(const double2 *__restri
     const long n = (long)ko0 * ko1 * h2;
     float bad = 0.0f, good = 0.0f;
     for (long t = (long)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += (long)gridDim.x * blockDim.x) {
-        const int kx = (int)(t % h2);
-        const int ky = (int)((t / h2) % ko1);
-        const int kz = (int)(t / ((long)h2 * ko1));
+        int kx, ky, kz;
+        if (n <= 0x7fffffffL) {
+            const unsigned u = (unsigned)t, r = u / (unsigned)h2;
+            kx = (int)(u - r * (unsigned)h2);
+            kz = (int)(r / (unsigned)ko1);
+            ky = (int)r - kz * ko1;
+        } else {
+            kx = (int)(t % h2);
+            ky = (int)((t / h2) % ko1);
+            kz = (int)(t / ((long)h2 * ko1));
+        }
         const double2 v = full[((long)kz * p1 + ky) * h2 + kx];
         out[6 * t] = (float)(v.x * inv); // component slot of `out` set by the caller
         bad = fmaxf(bad, (float)fabs(v.y));
@@ -733,7 +753,7 @@ int build_demag_kernel(DemagPlanImpl *P, bool keep_real)
     if (err == hipSuccess && newell) err = hipMalloc(&oct, sizeof(double) * 6 * ne);
     if (err == hipSuccess && newell) err = hipMalloc(&real64, sizeof(double) * Pn);
     if (err == hipSuccess) err = hipMalloc(&full, sizeof(double2) * (size_t)p[0] * p[1] * g.h2);
-    if (err == hipSuccess) err = hipMalloc(&stats, sizeof(unsigned int) * 16);
+    if (err == hipSuccess) err = hipMalloc(&stats, sizeof(unsigned int) * kStats * kStatStride);
     if (err != hipSuccess) {
         (void)hipFree(K6);
         (void)hipFree(oct);
@@ -745,9 +765,8 @@ int build_demag_kernel(DemagPlanImpl *P, bool keep_real)
     }
     do {
         if (K6 && hipMemset(K6, 0, sizeof(float) * 6 * Pn) != hipSuccess) { fail(MMX_ERR_HIP); break; }
-        if (hipMemset(stats, 0, sizeof(unsigned int) * 16) != hipSuccess) { fail(MMX_ERR_HIP); break; }
+        if (hipMemset(stats, 0, sizeof(unsigned int) * kStats * kStatStride) != hipSuccess) { fail(MMX_ERR_HIP); break; }
 
-        const int gb = 1024;
         if (newell) {
             NewellArgs a{};
             double dm = 0.0;
@@ -759,7 +778,7 @@ int build_demag_kernel(DemagPlanImpl *P, bool keep_real)
             a.rs2 = kNewellRSwitch * kNewellRSwitch * dm * dm;
             newell_rule5(a.t, a.w);
             newell_octant<<<dim3(div_up(ne, kBlock)), dim3(kBlock)>>>(a, oct);
-            maxabs_oct6<<<dim3(gb), dim3(kBlock)>>>(oct, ne, stats);
+            maxabs_oct6<<<dim3(stat_blocks(6 * ne, 256)), dim3(kBlock)>>>(oct, ne, stats);
             if (hipGetLastError() != hipSuccess) { set_error("newell_octant launch failed"); fail(MMX_ERR_HIP); break; }
         } else if (P->host_kernel) {
             // ConvPlan.loadKernel (convplan.go:85-115): the caller's kernel
@@ -769,7 +788,7 @@ int build_demag_kernel(DemagPlanImpl *P, bool keep_real)
                               hipMemcpyHostToDevice) != hipSuccess) { fail(MMX_ERR_HIP); break; }
             }
             if (rc) break;
-            maxabs_kernel<<<dim3(gb, 6), dim3(kBlock)>>>(K6, Pn, stats);
+            maxabs_kernel<<<dim3(stat_blocks(Pn, 256), 6), dim3(kBlock)>>>(K6, Pn, stats);
             if (hipGetLastError() != hipSuccess) { set_error("maxabs launch failed"); fail(MMX_ERR_HIP); break; }
         } else {
             // ranges of Kernel_Arne (kernel_magnetostatic.go:50-65)
@@ -806,14 +825,14 @@ int build_demag_kernel(DemagPlanImpl *P, bool keep_real)
                 if (hipGetLastError() != hipSuccess) { set_error("dex_combine launch failed"); fail(MMX_ERR_HIP); break; }
             }
             // IsZero test per component (maxwell_convolution.go:412-418)
-            maxabs_kernel<<<dim3(gb, 6), dim3(kBlock)>>>(K6, Pn, stats);
+            maxabs_kernel<<<dim3(stat_blocks(Pn, 256), 6), dim3(kBlock)>>>(K6, Pn, stats);
             if (hipGetLastError() != hipSuccess) { set_error("maxabs launch failed"); fail(MMX_ERR_HIP); break; }
         }
-        unsigned int hs[16];
+        unsigned int hs[kStats * kStatStride];
         if (hipMemcpy(hs, stats, sizeof(hs), hipMemcpyDeviceToHost) != hipSuccess) { fail(MMX_ERR_HIP); break; }
         float cmax[6], kmax = 0.0f;
         for (int c = 0; c < 6; c++) {
-            std::memcpy(&cmax[c], &hs[c], 4);
+            std::memcpy(&cmax[c], &hs[c * kStatStride], 4);
             kmax = fmaxf(kmax, cmax[c]);
         }
 
@@ -870,27 +889,27 @@ int build_demag_kernel(DemagPlanImpl *P, bool keep_real)
             if (p[0] > 1)
                 axis_fft_f64<<<dim3(div_up((long)nky * g.h2, wz), 1), dim3(kBlock), fft_f64_lds(p[0])>>>(
                     full, (long)p[1] * g.h2, (long)nky * g.h2, wz, f[0]);
-            extract_octant<<<dim3(1024), dim3(kBlock)>>>(full, p[1], g.ko0, g.ko1, g.h2, inv, dst,
-                                                         stats + 8, stats + 9);
+            extract_octant<<<dim3(stat_blocks(octant, 1024)), dim3(kBlock)>>>(full, p[1], g.ko0, g.ko1, g.h2, inv, dst,
+                                                         stats + 8 * kStatStride, stats + 9 * kStatStride);
             if (P->host_kernel) {
                 // components XX,YY,ZZ,YZ,XZ,XY: odd in axis 0 for XZ, XY; in axis 1 for YZ, XY
                 const int odd0 = (c == 4 || c == 5), odd1 = (c == 3 || c == 5);
                 octant_mirror_dev<<<dim3(1024), dim3(kBlock)>>>(full, p[0], p[1], g.h2, odd0, odd1,
-                                                                stats + 10);
+                                                                stats + 10 * kStatStride);
             }
             if (hipGetLastError() != hipSuccess) { set_error("kernel FFT launch failed"); fail(MMX_ERR_HIP); break; }
         }
         if (rc) break;
         if (hipMemcpy(hs, stats, sizeof(hs), hipMemcpyDeviceToHost) != hipSuccess) { fail(MMX_ERR_HIP); break; }
         float bad, good;
-        std::memcpy(&bad, &hs[8], 4);
-        std::memcpy(&good, &hs[9], 4);
+        std::memcpy(&bad, &hs[8 * kStatStride], 4);
+        std::memcpy(&good, &hs[9 * kStatStride], 4);
         P->bad_over_good = good > 0 ? (double)bad / (double)good : 0.0;
         if (P->host_kernel) {
             // ConvPlan only warns about imaginary parts (convplan.go:143-152);
             // the octant storage needs the mirror symmetry, so that is enforced
             float mdev;
-            std::memcpy(&mdev, &hs[10], 4);
+            std::memcpy(&mdev, &hs[10 * kStatStride], 4);
             if (good > 0 && (double)mdev / (double)good > 1e-5) {
                 set_error("convolution kernel: transformed kernel deviates from the mirror "
                           "symmetry of a demag/exchange kernel by %g of its maximum",

@@ -203,16 +203,16 @@ __device__ __forceinline__ void pair_epilogue(const DemagGeom &g, const FieldPar
     }
     if (MODE == EPI_CORR) {
         const float hh = 0.5f * io.h, mh = -0.5f * io.h;
-        float a0[3], a1[3];
-        float d = 0.0f;
+        float a0[3], a1[3], d0[3], d1[3];
 #pragma unroll
         for (int c = 0; c < 3; c++) {
             const float2 p = ld_off<float2>(io.tau0 + c * N, b0);
             a0[c] = m0[c] + (hh * t0[c] + mh * p.x);
             a1[c] = m1[c] + (hh * t1[c] + mh * p.y);
-            d = fmaxf(d, fmaxf(fabsf(t0[c] - p.x), fabsf(t1[c] - p.y)));
+            d0[c] = t0[c] - p.x;
+            d1[c] = t1[c] - p.y;
         }
-        errmax = fmaxf(errmax, (d != d) ? __builtin_inff() : d);
+        errmax = err_fold(err_fold(errmax, d0[0], d0[1], d0[2]), d1[0], d1[1], d1[2]);
         const float l0 = sqrtf(a0[0] * a0[0] + a0[1] * a0[1] + a0[2] * a0[2]);
         const float l1 = sqrtf(a1[0] * a1[0] + a1[1] * a1[1] + a1[2] * a1[2]);
         const float s0 = (ms.x == 0.0f) ? 0.0f : 1.0f, s1 = (ms.y == 0.0f) ? 0.0f : 1.0f;

@@ -568,8 +568,8 @@ sur_reduce_one(const float *__restrict__ part, int n, float *__restrict__ out)
 }
 
 // d loss / d out = 2 (out - target) / sum target^2 (bf16), *t2 = sum target^2;
-// the per-block partial sums of the squared error go to host_part (pinned
-// memory, at most kLossBlocks; a copy to pageable memory took 10 us), sum
+// the per-block partial sums of the squared error, in 64 bits, go to host_part
+// (pinned memory, at most kLossBlocks; a copy to pageable memory took 10 us), sum
 // target^2 behind them.  A wave takes 64 consecutive pixels and 4 of the 16
 // channels, so the target's planes are read in whole lines: 9.7 us with one
 // channel per thread, 6.6 us so at 256x256x4.
@@ -577,13 +577,13 @@ constexpr int kLossBlocks = 1024;
 __global__ void __launch_bounds__(kBlock)
 sur_loss(SurGeom s, const float *__restrict__ out, const float *__restrict__ bfine,
          const float *__restrict__ bc, const float *__restrict__ tgt_direct,
-         const float *__restrict__ t2, bf16_t *__restrict__ gout, float *__restrict__ host_part)
+         const float *__restrict__ t2, bf16_t *__restrict__ gout, double *__restrict__ host_part)
 {
-    __shared__ float red[kBlock / 64];
+    __shared__ double red[kBlock / 64];
     const long P = (long)s.n1 * s.n2;
     const int ch0 = 4 * __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nused = 3 * s.n0;
     const float gscale = 2.0f / fmaxf(*t2, 1e-30f);
-    float e2 = 0.0f;
+    double e2 = 0.0;
     for (long p = (long)blockIdx.x * 64 + (threadIdx.x & 63); p < P; p += (long)gridDim.x * 64) {
         const int y = (int)((unsigned)p / (unsigned)s.n2), x = (int)p - y * s.n2;
         const float4 o = *reinterpret_cast<const float4 *>(out + p * 16 + ch0);
@@ -593,7 +593,7 @@ sur_loss(SurGeom s, const float *__restrict__ out, const float *__restrict__ bfi
         for (int e = 0; e < 4; e++)
             if (ch0 + e < nused) {
                 const float d = ov[e] - target_at(s, bfine, bc, tgt_direct, p, y, x, ch0 + e);
-                e2 += d * d;
+                e2 += (double)d * (double)d;
                 g[e] = f2bf(gscale * d);
             }
         *reinterpret_cast<uint2 *>(gout + p * 16 + ch0) =
@@ -603,7 +603,7 @@ sur_loss(SurGeom s, const float *__restrict__ out, const float *__restrict__ bfi
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = e2;
     __syncthreads();
     if (threadIdx.x == 0) {
-        float s2 = 0.0f;
+        double s2 = 0.0;
         for (int w = 0; w < kBlock / 64; w++) s2 += red[w];
         host_part[blockIdx.x] = s2;
         if (blockIdx.x == 0) host_part[gridDim.x] = *t2;
@@ -681,7 +681,7 @@ struct mmx_surrogate {
     float *mc = nullptr, *bc = nullptr, *bfine = nullptr, *hd = nullptr;
     mmx::bf16_t *x0 = nullptr, *act[3] = {}, *gout = nullptr, *dz[3] = {};
     float *out = nullptr, *tgt = nullptr, *part = nullptr, *loss_part = nullptr;
-    float *loss_host = nullptr; // pinned: partial sums of the loss, then sum target^2
+    double *loss_host = nullptr; // pinned: partial sums of the loss, then sum target^2
     double *norm_part = nullptr;
     float *params = nullptr, *grads = nullptr, *adam_m = nullptr, *adam_v = nullptr;
     mmx::bf16_t *wt[4] = {}, *wbt[4] = {};
@@ -917,7 +917,7 @@ int mmx_surrogate_create(mmx_surrogate **sur, mmx_sim *sim, unsigned long long s
     if (rc == MMX_OK) rc = dalloc(&S->tgt, P * 3 * n0);
     if (rc == MMX_OK) rc = dalloc(&S->part, (size_t)4 * grad_parts(n1, n2) * kSurSlot);
     if (rc == MMX_OK) rc = dalloc(&S->loss_part, P / 16 + 1);
-    if (rc == MMX_OK && hipHostMalloc(&S->loss_host, sizeof(float) * (loss_blocks(P) + 1)) != hipSuccess) {
+    if (rc == MMX_OK && hipHostMalloc(&S->loss_host, sizeof(double) * (loss_blocks(P) + 1)) != hipSuccess) {
         set_error("surrogate: cannot allocate pinned memory");
         rc = MMX_ERR_NOMEM;
     }

@@ -397,18 +397,22 @@ __device__ __forceinline__ void wgrad_tiles(const bf16_t *__restrict__ x, const 
                 acc[3 * d + 2] = mfma_k32(a, __builtin_bit_cast(sh8, b2), acc[3 * d + 2]);
             }
         }
-        // bias gradient: wave w sums pixels 64 w .. 64 w + 63 of channel `lane`
+        // bias gradient: wave w sums pixels 64 w .. 64 w + 63 of channel `lane`,
+        // tile by tile (one chain over all tiles would round each pixel to the
+        // running total)
         if (lane < COUT) {
+            float part = 0.0f;
 #pragma unroll
             for (int p = 0; p < 64; p += 8) {
                 const uint4 w = *reinterpret_cast<const uint4 *>(dzt + lane * kWgD + 64 * wave + p);
                 const unsigned e[4] = {w.x, w.y, w.z, w.w};
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
-                    sum += bf2f((bf16_t)(e[i] & 0xffffu));
-                    sum += bf2f((bf16_t)(e[i] >> 16));
+                    part += bf2f((bf16_t)(e[i] & 0xffffu));
+                    part += bf2f((bf16_t)(e[i] >> 16));
                 }
             }
+            sum += part;
         }
     }
     // D[m = co][n = ci]: lane holds co = mt*16 + kq + e, ci = nt*16 + n

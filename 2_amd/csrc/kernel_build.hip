@@ -289,7 +289,8 @@ static void arne_reach(ArneArgs &a)
 {
     const int most[3] = {a.x2 > -a.x1 ? a.x2 : -a.x1, a.y2 > -a.y1 ? a.y2 : -a.y1,
                          a.z2 > -a.z1 ? a.z2 : -a.z1};
-    const double far = a.accuracy * fmax(a.cell[0], fmax(a.cell[1], a.cell[2])) / 1.5;
+    // (finite, so that the loop ends for any cell)
+    const double far = fmin(a.accuracy * fmax(a.cell[0], fmax(a.cell[1], a.cell[2])) / 1.5, 1e300);
     for (double d = far;; d *= 0.8) {
         double count = 1.0;
         for (int c = 0; c < 3; c++) {

@@ -82,8 +82,12 @@ yi_kernel(DemagGeom g, LineFFT<float> fy, int W, const float2 *__restrict__ yb,
 
 // ------------------------------------------------- XI pass (+ fused epilogue)
 
+// Six waves per SIMD: the direct DFTs of a long prime wait for their loads, and
+// the epilogue, whose loads all come first, took registers for five or four
+// (31x127x127 torque 13.05 ms with one load at a time, 14.45 ms so unbounded,
+// 13.18 ms bounded, with 4 to 12 registers spilled; 34x34 films 115, 104, 108 us).
 template <int MODE>
-__global__ void __launch_bounds__(kBlock)
+__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6)))
 xi_kernel(DemagGeom g, LineFFT<float> fx, int RB, const float2 *__restrict__ xb,
           FieldParams fp, EpilogueIO io)
 {

@@ -37,8 +37,8 @@ def _check(mmx, n, pbc=(0, 0, 0), masked=False):
     assert np.abs(b.cpu().numpy() - want).max() <= 4e-6 * np.abs(want).max()
 
 
-# x half-lengths: one radix each, two stages of the larger class on many rows,
-# three stages, primes 11 and 13, an odd length
+# x half-lengths: one stage, two and three stages of radices up to 16 (which is
+# what few rows take), 25 x 25, primes 11 and 13, odd lengths
 X = [3, 7, 9, 11, 13, 15, 18, 20, 21, 22, 25, 26, 27, 28, 30, 33, 39, 42, 44, 45, 50, 60, 63, 65, 66, 75, 77, 78, 81,
      88, 90, 91, 99, 100, 104, 110, 117, 120, 121, 125, 130, 143, 150, 156, 169, 176, 195, 200, 208, 210, 225, 240,
      250, 270, 286, 300, 343, 360, 375, 420, 500, 600, 625, 729, 1000]
@@ -110,8 +110,8 @@ def test_batch_tiles(mmx, grids):
 
 # grids of more rows than workgroups wanted: the two-cell epilogue with uniform
 # parameters and with maps, and the per-cell one with the spin-transfer torque,
-# on lengths of either register class; the corrector's maximum over many
-# workgroups
+# on radices up to 16 (above: test_cells_in_pairs_large_radix); the corrector's
+# maximum over many workgroups
 @pytest.mark.parametrize("maps", [False, True])
 @pytest.mark.parametrize("zl", [False, True])
 @pytest.mark.parametrize("n,pbc", [((11, 100, 24), (0, 0, 0)), ((2, 650, 22), (0, 0, 1)), ((3, 350, 9), (0, 1, 0))])
@@ -149,3 +149,55 @@ def test_cells_in_pairs(mmx, n, pbc, zl, maps):
     e_gpu, e_orc = sim.try_step(1e-15), prob.try_step(mo, 1e-15)
     assert abs(e_gpu - e_orc) <= 1e-4 * e_orc
     assert np.abs(sim.getarray("m") - prob.normalized(mo)).max() <= 1e-5
+
+
+# the class of radices above 16: every one of them in y, in a film's y and in z,
+# and those that x uses on grids of more than 2048 rows
+LARGE_RADIX = {324: (18, 18), 400: (20, 20), 294: (21, 14), 484: (22, 22), 768: (32, 24), 350: (25, 14),
+               676: (26, 26), 594: (27, 22), 784: (28, 28), 900: (30, 30)}
+LARGE_RADIX_X = {162: (18, 9), 200: (20, 10), 147: (21, 7), 242: (22, 11), 312: (24, 13), 125: (25, 5),
+                 338: (26, 13), 243: (27, 9), 392: (28, 14)}
+
+
+def _radices(L, top2):
+    """The rule of comp_plan (comp_x.hip) over the radices of comp_fft.hpp: two
+    stages, else three, with the smallest largest radix."""
+    have = _compiled_radices()
+    two = [(L // r1, r1) for r1 in range(1, top2 + 1)
+           if L % r1 == 0 and r1 <= L // r1 <= top2 and {r1, L // r1} <= have]
+    if two:
+        return min(two)
+    three = [(L // r1 // r2, r1, r2) for r2 in range(2, 33) for r1 in range(r2, 33)
+             if L % (r1 * r2) == 0 and L // r1 // r2 >= r1 and {r1, r2, L // r1 // r2} <= have]
+    return min(three) if three else ()
+
+
+def _compiled_radices():
+    import os
+    import re
+    src = open(os.path.join(os.path.dirname(__file__), "..", "2_amd", "csrc", "comp_fft.hpp")).read()
+    lists = re.findall(r"#define MMX_COMP_RADICES_\d+\(X\)[^\n]*\n([^\n]*)", src)
+    return {int(r) for text in lists for r in re.findall(r"X\((\d+)\)", text)}
+
+
+@pytest.mark.parametrize("L", sorted(LARGE_RADIX))
+@pytest.mark.parametrize("axis", ["y", "film", "z"])
+def test_large_radices(mmx, L, axis):
+    assert _radices(L, 32) == LARGE_RADIX[L]
+    k = L // 2
+    _check(mmx, {"y": (2, k, 5), "film": (1, k, 5), "z": (k, 3, 5)}[axis])
+
+
+@pytest.mark.parametrize("Lx", sorted(LARGE_RADIX_X))
+def test_large_radices_x(mmx, Lx):
+    assert _radices(Lx, 32) == LARGE_RADIX_X[Lx]
+    _check(mmx, (1, 2100, 2 * Lx), (0, 1, 1))
+
+
+# the epilogues in the larger class: fields, first stage and corrector
+@pytest.mark.parametrize("maps", [False, True])
+@pytest.mark.parametrize("zl", [False, True])
+def test_cells_in_pairs_large_radix(mmx, zl, maps):
+    n = (3, 700, 162)
+    assert _radices(n[2], 32) == (18, 9) and n[0] * n[1] > 2048
+    test_cells_in_pairs(mmx, n, (0, 0, 0), zl, maps)

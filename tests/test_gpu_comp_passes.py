@@ -201,3 +201,30 @@ def test_cells_in_pairs_large_radix(mmx, zl, maps):
     n = (3, 700, 162)
     assert _radices(n[2], 32) == (18, 9) and n[0] * n[1] > 2048
     test_cells_in_pairs(mmx, n, (0, 0, 0), zl, maps)
+
+
+# arrays that start off an 8-byte boundary take one cell at a time: the same bits
+@pytest.mark.parametrize("n", [(2, 520, 20), (1, 6, 100)])
+def test_arrays_off_the_pair_boundary(mmx, n):
+    import torch
+    print("unaligned", n, flush=True)
+    plan = mmx.DemagPlan(n, (3e-9, 4e-9, 4e-9))
+    rng = np.random.default_rng(n[1])
+    N = int(np.prod(n))
+    src = [rng.standard_normal(3 * N).astype(np.float32), rng.uniform(0.5, 1.5, N).astype(np.float32)]
+
+    def field(om, ob, os_):
+        m, s = (torch.zeros(a.size + 2, device="cuda") for a in src)
+        b = torch.full((3 * N + 2,), np.nan, device="cuda")
+        m[om:om + 3 * N] = torch.from_numpy(src[0]).cuda()
+        s[os_:os_ + N] = torch.from_numpy(src[1]).cuda()
+        assert m.data_ptr() % 8 == b.data_ptr() % 8 == s.data_ptr() % 8 == 0
+        plan.update_b(b.data_ptr() + 4 * ob, m.data_ptr() + 4 * om, 8e5, s.data_ptr() + 4 * os_, None)
+        torch.cuda.synchronize()
+        out = b.cpu().numpy()
+        assert np.isnan(out[:ob]).all() and np.isnan(out[ob + 3 * N:]).all()
+        return out[ob:ob + 3 * N]
+    want = field(0, 0, 0)
+    assert np.isfinite(want).all()
+    for off in ((1, 0, 0), (0, 1, 0), (0, 0, 1), (1, 1, 1)):
+        assert np.array_equal(field(*off), want)

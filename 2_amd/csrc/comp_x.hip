@@ -25,7 +25,7 @@ CompFFT comp_plan(int L, const LineFFT<float> &f, int top2)
     c.tw = f.tw;
     c.rtw = f.rtw;
     int top = top2 + 1;
-    // two stages, the larger radix first (the z pass keeps 3 R1 points per thread)
+    // two stages, the larger radix first
     for (int r1 = 1; r1 <= top2; r1++) {
         const int r0 = L / r1;
         if (L % r1 || r0 < r1 || !comp_radix(r0) || !comp_radix(r1) || r0 >= top) continue;

@@ -103,7 +103,7 @@ int fast_y2d_as_z(const DemagPlanImpl *P, hipStream_t st)
     switch (f.p0) {
 #define CASE(L)                                                                              \
     case L: return z_len_geom<L>(f, P->fy.tw, P->kern, P->xbuf, st);
-        MMX_SHORT_LENGTHS(CASE)
+        MMX_FILM_LENGTHS(CASE)
 #undef CASE
     default: set_error("fast_y2d_as_z: length %d", f.p0); return MMX_ERR_SIZE;
     }

@@ -36,7 +36,7 @@ template <int LX> struct RowTile {
     static constexpr int T = Split<LX>::T;
     static constexpr int E = Split<LX>::E;
     static constexpr int G = E / T;
-    static constexpr int R = (LX == 2048) ? 4 : (LX == 1024 ? 8 : 256 / T);
+    static constexpr int R = (LX == 1024) ? 8 : 256 / T;
     // pitch = 1 mod 32 complex: the transposed reads of 16-32 rows x T lanes
     // hit distinct bank pairs
     static constexpr int S = T * R + 1;
@@ -780,7 +780,8 @@ int xi_len(const DemagPlanImpl *P, int mode, const FieldParams &fp, const Epilog
 // fast_odd_short, fast_odd_long)
 #define MMX_X_LENGTHS(X) X(8) X(16) X(32) X(64) X(128) X(256)
 #define MMX_XF_LENGTHS(X) MMX_X_LENGTHS(X) X(1024)
-#define MMX_POW2_LENGTHS(X) X(8) X(16) X(32) X(64) X(128) X(256) X(512) X(1024) X(2048)
+#define MMX_POW2_FILM(X) X(8) X(16) X(32) X(64) X(128) X(256) X(512) X(1024)
+#define MMX_POW2_LENGTHS(X) MMX_POW2_FILM(X) X(2048)
 #define MMX_R3_SHORT(X) X(24) X(48) X(96) X(192)
 #define MMX_R5_SHORT(X) X(40) X(80)
 #define MMX_R7_SHORT(X) X(56) X(112)
@@ -788,6 +789,7 @@ int xi_len(const DemagPlanImpl *P, int mode, const FieldParams &fp, const Epilog
 #define MMX_R5_LONG(X) X(160) X(320)
 #define MMX_R7_LONG(X) X(224) X(448)
 #define MMX_SHORT_LENGTHS(X) MMX_POW2_LENGTHS(X) MMX_R3_SHORT(X) MMX_R5_SHORT(X) MMX_R7_SHORT(X)
+#define MMX_FILM_LENGTHS(X) MMX_POW2_FILM(X) MMX_R3_SHORT(X) MMX_R5_SHORT(X) MMX_R7_SHORT(X)
 #define MMX_ALL_LENGTHS(X) MMX_SHORT_LENGTHS(X) MMX_R3_LONG(X) MMX_R5_LONG(X) MMX_R7_LONG(X)
 
 } // namespace mmx

@@ -145,8 +145,8 @@ int xi_len(const DemagPlanImpl *P, int mode, const FieldParams &fp, const Epilog
 #define MMX_INST_Y(L)                                                                        \
     template int yf_len<L>(const DemagPlanImpl *, hipStream_t);                              \
     template int yi_len<L>(const DemagPlanImpl *, hipStream_t);
-#define MMX_INST_Z(L)                                                                        \
-    template int z_len<L>(const DemagPlanImpl *, hipStream_t);                               \
+#define MMX_INST_Z(L) template int z_len<L>(const DemagPlanImpl *, hipStream_t);
+#define MMX_INST_FILM(L)                                                                     \
     template int z_len_geom<L>(const DemagGeom &, const float2 *, const float *, float2 *,   \
                                hipStream_t);
 #define MMX_INST_XI(L, VAR)                                                                  \

@@ -7,6 +7,7 @@
 namespace mmx {
 
 MMX_R3_SHORT(MMX_INST_Z)
+MMX_R3_SHORT(MMX_INST_FILM)
 MMX_R3_SHORT(MMX_INST_Y)
 MMX_R3_LONG(MMX_INST_Y)
 

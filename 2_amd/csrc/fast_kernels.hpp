@@ -181,8 +181,8 @@ yi_fast(DemagGeom g, int ntx, const float2 *__restrict__ tw, const float2 *__res
 // of four waves per CU; the 32 lanes of a b64 access hit distinct bank pairs in
 // both directions (T W + 2 W = 2 W mod 32).  SPLIT, 8 columns (64-byte row
 // segments): real and imaginary parts cross one after the other through a
-// buffer of floats, which leaves room for four waves per SIMD (128 registers)
-// at the price of three more barriers; the 64 lanes of a b32 access hit distinct
+// buffer of floats, which leaves room for four waves per SIMD (128 registers,
+// 8 or 9 of them spilled) at the price of three more barriers; the 64 lanes of a b32 access hit distinct
 // banks (T W + 2 W = 2 W mod 64).
 //
 // yi takes the split tile when that gives every CU a workgroup

@@ -353,10 +353,9 @@ __device__ inline void block_max_to(float v, unsigned int *dst)
 }
 
 // The corrector's error maximum: workgroup b merges into word b & mask (0: one
-// word),
-// each in a cache line of its own (atomics on one word run one after another,
-// about 10 ns each: 1000 workgroups of a 200x200x5 corrector spent 10 of its 23
-// us there).  The maximum of all slots is the result.
+// word), each in a cache line of its own (atomics on one word run one after
+// another, about 10 ns each: 1000 workgroups of a 200x200x5 corrector spent 10 of
+// its 23 us there).  The maximum of all slots is the result.
 constexpr int kErrSlots = 64, kErrStride = 16;
 
 __device__ inline void block_max_slot(float v, unsigned int *slots, unsigned int mask)

@@ -299,8 +299,11 @@ inline bool fast_odd_long(int L) { return L == 384 || L == 160 || L == 320 || L 
 // at 512 points and more, and at the lengths with an odd factor, one wave per
 // SIMD is left and the composite-radix passes win (xf / xi at 192x192x48: 28 /
 // 55 against 28 / 37 us, 512x512x16: 59 / 101 against 54 / 92, 2048x128x64: 619 /
-// 1477 against 301 / 452), but for xf at 1024 points without a map (1024x1024x32:
-// 405 against 441 us).
+// 1477 against 301 / 452), but for xf at 1024 points without a map (register
+// against composite-radix us, x points first: 1024x512x4 28.5 / 33.3, 1024x1000x8
+// 106.5 / 108, 1024x256x64 207 / 224, 1024x1024x32 404 / 448).  With a map its
+// threads hold more and it loses from 1024x1000x8 on (127 / 114, 262 / 231, 536 /
+// 457; 1024x512x4 32.3 / 34.0).
 inline bool fast_x_length_impl(int L)
 {
     return L == 8 || L == 16 || L == 32 || L == 64 || L == 128 || L == 256;

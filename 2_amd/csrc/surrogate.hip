@@ -146,12 +146,13 @@ __device__ __forceinline__ float input_channel(const SurGeom &s, const float *__
     return 0.0f;
 }
 
-// Packed bf16 input [P][32] (used by training and the tests; inference packs
-// inside the first convolution).  Bound by the latency of its scattered plane
+// Packed bf16 input [P][32].  Bound by the latency of its scattered plane
 // reads: a wave takes 64 consecutive pixels and 8 channels, so every plane is
 // read in whole lines and a pixel's 8 channels leave in one 16-byte store
 // (256x256x4: 12.6 us with one channel per thread, which read 4 pixels of 16
-// planes per wave, 8.0 us so).
+// planes per wave, 8.0 us so).  A first convolution that forms its input itself
+// reads them by pixel: 25.9 us (21.1 with 4 channels per thread) against 8.1 for
+// this and 5.7 for the convolution of the packed input.
 __global__ void __launch_bounds__(kBlock)
 sur_pack(SurGeom s, const float *__restrict__ m, const float *__restrict__ bc,
          bf16_t *__restrict__ x0)
@@ -183,8 +184,7 @@ __device__ __forceinline__ fl4 mfma_any(sh4 a, sh4 b, fl4 c)
 // over a 16 x 8 pixel tile per workgroup of 4 waves.  The MFMA computes
 // D = A B with A = weights (rows co, k = ci) and B = the input (k = ci,
 // columns = 16 pixels of a row), so each lane ends up holding 4 consecutive
-// output channels of one pixel.  PACK: the input is formed from (m, coarse B)
-// instead of being read from `in`.
+// output channels of one pixel.
 //
 // Bound by the latency of one load - LDS - MFMA chain per workgroup (512
 // workgroups at 256x256, two per CU), not by the 36 MFMA of a wave.  A wave
@@ -193,11 +193,11 @@ __device__ __forceinline__ fl4 mfma_any(sh4 a, sh4 b, fl4 c)
 // fragment read once from LDS serves the three output rows it belongs to.
 // With the weights staged in LDS (18 KB per workgroup) and every fragment read
 // per output row: 9.0 us a layer at 256x256, so 5.6 us.
-template <int CIN, int COUT, int EPI, int PACK>
+template <int CIN, int COUT, int EPI>
 __global__ void __launch_bounds__(kBlock)
 sur_conv(const bf16_t *__restrict__ in, const bf16_t *__restrict__ wt,
          const float *__restrict__ bias, const bf16_t *__restrict__ mask, void *__restrict__ out,
-         int H, int W, SurGeom s, const float *__restrict__ m, const float *__restrict__ bc)
+         int H, int W)
 {
     static_assert(CIN == 32 || CIN == 16, "one MFMA per tap");
     using Frag = std::conditional_t<CIN == 32, sh8, sh4>;
@@ -217,18 +217,8 @@ sur_conv(const bf16_t *__restrict__ in, const bf16_t *__restrict__ wt,
         const int q = t % NQ, pc = t / NQ, cx = pc % 18, cy = pc / 18;
         const int gy = y0 + cy - 1, gx = x0 + cx - 1;
         u[i] = uint4{0u, 0u, 0u, 0u};
-        if (t < TASKS && gy >= 0 && gy < H && gx >= 0 && gx < W) {
-            if (PACK) {
-                unsigned w[4];
-#pragma unroll
-                for (int e = 0; e < 4; e++)
-                    w[e] = (unsigned)f2bf(input_channel(s, m, bc, gy, gx, 8 * q + 2 * e)) |
-                           ((unsigned)f2bf(input_channel(s, m, bc, gy, gx, 8 * q + 2 * e + 1)) << 16);
-                u[i] = uint4{w[0], w[1], w[2], w[3]};
-            } else {
-                u[i] = *reinterpret_cast<const uint4 *>(in + ((long)gy * W + gx) * CIN + 8 * q);
-            }
-        }
+        if (t < TASKS && gy >= 0 && gy < H && gx >= 0 && gx < W)
+            u[i] = *reinterpret_cast<const uint4 *>(in + ((long)gy * W + gx) * CIN + 8 * q);
     }
     Frag a[9];
 #pragma unroll
@@ -738,24 +728,22 @@ int prep_weights(mmx_surrogate *S, hipStream_t st)
     return MMX_OK;
 }
 
-// the net on a packed input (PACK = 0) or formed from (m, coarse B)
-int net_forward(mmx_surrogate *S, bool pack, const float *m, hipStream_t st)
+// the net on the packed input S->x0, formed from (m, coarse B) first where m is given
+int net_forward(mmx_surrogate *S, const float *m, hipStream_t st)
 {
     const dim3 grid(S->W / 16, S->H / 8), blk(kBlock);
     const float *b[4] = {S->params + S->off_b[0], S->params + S->off_b[1], S->params + S->off_b[2],
                          S->params + S->off_b[3]};
-    if (pack)
-        sur_conv<32, 32, CE_RELU_BF16, 1><<<grid, blk, 0, st>>>(nullptr, S->wt[0], b[0], nullptr,
-                                                                S->act[0], S->H, S->W, S->s, m, S->bc);
-    else
-        sur_conv<32, 32, CE_RELU_BF16, 0><<<grid, blk, 0, st>>>(S->x0, S->wt[0], b[0], nullptr,
-                                                                S->act[0], S->H, S->W, S->s, nullptr, nullptr);
-    sur_conv<32, 32, CE_RELU_BF16, 0><<<grid, blk, 0, st>>>(S->act[0], S->wt[1], b[1], nullptr,
-                                                            S->act[1], S->H, S->W, S->s, nullptr, nullptr);
-    sur_conv<32, 32, CE_RELU_BF16, 0><<<grid, blk, 0, st>>>(S->act[1], S->wt[2], b[2], nullptr,
-                                                            S->act[2], S->H, S->W, S->s, nullptr, nullptr);
-    sur_conv<32, 16, CE_LINEAR_F32, 0><<<grid, blk, 0, st>>>(S->act[2], S->wt[3], b[3], nullptr,
-                                                             S->out, S->H, S->W, S->s, nullptr, nullptr);
+    if (m)
+        sur_pack<<<dim3((unsigned)div_up(S->P, 64)), dim3(kBlock), 0, st>>>(S->s, m, S->bc, S->x0);
+    sur_conv<32, 32, CE_RELU_BF16><<<grid, blk, 0, st>>>(S->x0, S->wt[0], b[0], nullptr, S->act[0], S->H,
+                                                         S->W);
+    sur_conv<32, 32, CE_RELU_BF16><<<grid, blk, 0, st>>>(S->act[0], S->wt[1], b[1], nullptr, S->act[1],
+                                                         S->H, S->W);
+    sur_conv<32, 32, CE_RELU_BF16><<<grid, blk, 0, st>>>(S->act[1], S->wt[2], b[2], nullptr, S->act[2],
+                                                         S->H, S->W);
+    sur_conv<32, 16, CE_LINEAR_F32><<<grid, blk, 0, st>>>(S->act[2], S->wt[3], b[3], nullptr, S->out,
+                                                          S->H, S->W);
     MMX_CHECK_LAUNCH();
     return MMX_OK;
 }
@@ -777,11 +765,11 @@ int net_backward(mmx_surrogate *S, const float *tgt_direct, float lr, double *lo
     sur_loss<<<dim3(nlb), dim3(kBlock), 0, st>>>(S->s, S->out, S->bfine, S->bc, tgt_direct, t2,
                                                  S->gout, S->loss_host);
     const dim3 grid(S->W / 16, S->H / 8), blk(kBlock);
-    sur_conv<16, 32, CE_MASK_BF16, 0><<<grid, blk, 0, st>>>(S->gout, S->wbt[3], nullptr, S->act[2],
-                                                            S->dz[2], S->H, S->W, S->s, nullptr, nullptr);
+    sur_conv<16, 32, CE_MASK_BF16><<<grid, blk, 0, st>>>(S->gout, S->wbt[3], nullptr, S->act[2], S->dz[2],
+                                                         S->H, S->W);
     for (int l = 2; l > 0; l--)
-        sur_conv<32, 32, CE_MASK_BF16, 0><<<grid, blk, 0, st>>>(
-            S->dz[l], S->wbt[l], nullptr, S->act[l - 1], S->dz[l - 1], S->H, S->W, S->s, nullptr, nullptr);
+        sur_conv<32, 32, CE_MASK_BF16><<<grid, blk, 0, st>>>(S->dz[l], S->wbt[l], nullptr, S->act[l - 1],
+                                                             S->dz[l - 1], S->H, S->W);
     // weight gradients of all layers from the kept inputs and output gradients
     const SurLayers ly = sur_layers(S);
     const int ntile = (S->W / 16) * (S->H / 16), nparts = grad_parts(S->H, S->W);
@@ -835,7 +823,7 @@ int surrogate_eval(mmx_surrogate *S, int mode, const float *m0, const float *tau
 {
     const float *m = tau0 ? mpred : m0;
     MMX_TRY(coarse_field(S, m0, tau0, h, mpred, st));
-    MMX_TRY(net_forward(S, true, m, st));
+    MMX_TRY(net_forward(S, m, st));
     const DemagGeom &g = S->sim->plan->impl.g;
     const int nb = (int)div_up(S->s.N, kBlock);
     switch (mode) {
@@ -1023,7 +1011,7 @@ int mmx_surrogate_net(mmx_surrogate *sur, const float *x_host, const float *tgt_
         else xb[e] = (unsigned short)((u + 0x7fffu + ((u >> 16) & 1u)) >> 16);
     }
     MMX_HIP(hipMemcpyAsync(S->x0, xb.data(), sizeof(unsigned short) * P * 32, hipMemcpyHostToDevice, st));
-    MMX_TRY(net_forward(S, false, nullptr, st));
+    MMX_TRY(net_forward(S, nullptr, st));
     if (tgt_host) {
         MMX_HIP(hipMemcpyAsync(S->tgt, tgt_host, sizeof(float) * P * 3 * S->s.n0, hipMemcpyHostToDevice, st));
         MMX_TRY(net_backward(S, S->tgt, 0.0f, loss, st));
@@ -1045,9 +1033,7 @@ int mmx_surrogate_train_step(mmx_surrogate *sur, const float *m_dev, float lr, d
     MMX_TRY(mmx_demag_update_b(x->plan, S->bfine, S->bfine + N, S->bfine + 2 * N, m_dev, m_dev + N,
                                m_dev + 2 * N, nullptr, (float)x->msat, st));
     MMX_TRY(coarse_field(S, m_dev, nullptr, 0.0f, nullptr, st));
-    sur_pack<<<dim3((unsigned)div_up(S->P, 64)), dim3(kBlock), 0, st>>>(S->s, m_dev, S->bc, S->x0);
-    MMX_CHECK_LAUNCH();
-    MMX_TRY(net_forward(S, false, nullptr, st));
+    MMX_TRY(net_forward(S, m_dev, st));
     return net_backward(S, nullptr, lr, loss, st);
 }
 
@@ -1060,7 +1046,7 @@ int mmx_surrogate_predict_b(mmx_surrogate *sur, const float *m_dev, float *b_dev
     if (coarse_only) {
         MMX_HIP(hipMemsetAsync(S->out, 0, sizeof(float) * S->P * 16, st));
     } else {
-        MMX_TRY(net_forward(S, true, m_dev, st));
+        MMX_TRY(net_forward(S, m_dev, st));
     }
     const DemagGeom &g = S->sim->plan->impl.g;
     const FieldParams fp = sim_field_params(S->sim);
